@@ -281,7 +281,6 @@ int prox_entry(int op_in, int data_in, int result_in, int64_t m, int64_t n, cons
 
   const bool reg_ok = m <= kRegMaxM;
   const bool topk = op == SDCA_PROX_TOPK_SIMPLEX || op == SDCA_PROX_TOPK_CONE;
-  const bool knap = op == SDCA_PROX_KNAPSACK_EQ || op == SDCA_PROX_KNAPSACK_LE;
   // The biased simplex, cone and knapsack run in the register kernel;
   // columns whose search needs more of the sorted column are deferred to the
   // workgroup-per-column kernel through the column list.
@@ -430,7 +429,7 @@ int prox_entry(int op_in, int data_in, int result_in, int64_t m, int64_t n, cons
     SDCA_HIP_TRY(launch_two_ent(a), "two_entropy kernel (wave per column)");
   } else if (ent_biased) {
     SDCA_HIP_TRY(launch_ent_biased(a), "topk_entropy_biased kernel (wave per column)");
-  } else if ((topk || knap || reg_biased) && (!reg_ok || (topk_like && p.k > kTopkMaxK))) {
+  } else if (topk_like && (!reg_ok || p.k > kTopkMaxK)) {
     // Columns beyond the register kernel: one workgroup per sorted column.
     SDCA_HIP_TRY(launch_slow(a, true), "prox kernel (workgroup per column)");
   } else {

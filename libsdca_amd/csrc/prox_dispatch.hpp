@@ -82,7 +82,9 @@ hipError_t launch_one(const ProxLaunch& a) {
 // Columns above kRegMaxM rows: one workgroup per column (kWideThreads
 // threads, kMaxWideThreads for the largest fp32 columns), C slots per
 // thread; the column (at most kMaxColumnBytes) is staged in LDS and the
-// group reductions combine the waves through LDS.
+// group reductions combine the waves through LDS.  (The knapsack, 40e6 fp32
+// entries: m = 3000 144 us, 8000 88, 16000 105, 30000 160, against 2286,
+// 2495, 4893 and 11745 with the column sorted in LDS.)
 template <int FAM, int KM, class D, class R>
 hipError_t launch_wide(const ProxLaunch& a) {
   constexpr int G = kWideThreads, G2 = kMaxWideThreads;
@@ -98,9 +100,8 @@ hipError_t launch_wide(const ProxLaunch& a) {
 // m = 200 on eight).
 template <int FAM, int KM, class D, class R>
 hipError_t launch_by_m(const ProxLaunch& a) {
-  // The knapsack and top-k families take the sorted-column kernel above
-  // kRegMaxM rows.
-  if constexpr (FAM == FAM_ENT || FAM == FAM_TOPKENT || FAM == FAM_TWO) {
+  // The top-k family takes the sorted-column kernel above kRegMaxM rows.
+  if constexpr (FAM != FAM_TOPK) {
     if (a.m > kRegMaxM) return launch_wide<FAM, KM, D, R>(a);
   }
   // The knapsack family's smallest columns (C1: m = 10) in exactly ten

@@ -429,9 +429,13 @@ int prox_entry(int op_in, int data_in, int result_in, int64_t m, int64_t n, cons
     SDCA_HIP_TRY(launch_two_ent(a), "two_entropy kernel (wave per column)");
   } else if (ent_biased) {
     SDCA_HIP_TRY(launch_ent_biased(a), "topk_entropy_biased kernel (wave per column)");
-  } else if (topk_like && (!reg_ok || p.k > kTopkMaxK)) {
-    // Columns beyond the register kernel: one workgroup per sorted column.
-    SDCA_HIP_TRY(launch_slow(a, true), "prox kernel (workgroup per column)");
+  } else if (topk_like && !topk_in_registers(op, data, m, p.k)) {
+    // Columns beyond the register kernel: by selection, or for the largest
+    // k one workgroup per sorted column.
+    if (select_supported(a))
+      SDCA_HIP_TRY(launch_select(a, true), "prox kernel (selection)");
+    else
+      SDCA_HIP_TRY(launch_slow(a), "prox kernel (workgroup per column)");
   } else {
     // Deferred-column list: [count, done, column ids...].  The deferred-column
     // kernel zeroes both counters when its last workgroup finishes, so a
@@ -474,7 +478,8 @@ int prox_entry(int op_in, int data_in, int result_in, int64_t m, int64_t n, cons
       SDCA_HIP_TRY(launch_two_sort(a, false), "two_simplex_sort kernel (deferred columns)");
       wsr->list_zeroed = true;
     } else if (listed) {
-      SDCA_HIP_TRY(launch_slow(a, false), "prox kernel (deferred columns)");
+      // (the biased knapsack defers nothing: its list stays empty)
+      if (topk_like) SDCA_HIP_TRY(launch_select(a, false), "prox kernel (deferred columns)");
       wsr->list_zeroed = true;
     }
   }

@@ -100,7 +100,7 @@ hipError_t launch_wide(const ProxLaunch& a) {
 // m = 200 on eight).
 template <int FAM, int KM, class D, class R>
 hipError_t launch_by_m(const ProxLaunch& a) {
-  // The top-k family takes the sorted-column kernel above kRegMaxM rows.
+  // The top-k family's columns above 1024 rows go by selection.
   if constexpr (FAM != FAM_TOPK) {
     if (a.m > kRegMaxM) return launch_wide<FAM, KM, D, R>(a);
   }
@@ -117,8 +117,15 @@ hipError_t launch_by_m(const ProxLaunch& a) {
   if (a.m <= 200) return launch_one<FAM, KM, D, R, 8, 25>(a);
   if (a.m <= 256) return launch_one<FAM, KM, D, R, 16, 16>(a);
   if (a.m <= 512) return launch_one<FAM, KM, D, R, 16, 32>(a);
-  if (a.m <= 1024) return launch_one<FAM, KM, D, R, 64, 16>(a);
-  return launch_one<FAM, KM, D, R, 64, 32>(a);
+  if constexpr (FAM == FAM_TOPK) {
+    if constexpr (sizeof(D) == 4 && KM != 15) {
+      if (a.m <= 1024) return launch_one<FAM, KM, D, R, 64, 16>(a);
+    }
+    return hipErrorInvalidValue;
+  } else {
+    if (a.m <= 1024) return launch_one<FAM, KM, D, R, 64, 16>(a);
+    return launch_one<FAM, KM, D, R, 64, 32>(a);
+  }
 }
 
 template <int FAM, int KM>

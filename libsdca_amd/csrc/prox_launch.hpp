@@ -42,9 +42,17 @@ constexpr int64_t kMaxColumnBytes = 128 * 1024;
 inline int64_t max_rows(int data) {
   return kMaxColumnBytes / (data == SDCA_F32 ? 4 : 8);
 }
-// Top-k operators keep k <= kTopkMaxK in registers; larger k takes the
-// workgroup-per-column kernel.
-constexpr int64_t kTopkMaxK = 8;
+// Whether the register kernel takes a top-k operator's columns: its sorted
+// lists hold k <= 8 of a column (k <= 15 with the longest list, which pays
+// where several columns share a wave: 40e6 fp32 entries of m = 100, k = 10,
+// 563 us by selection, one wave per column).  On columns with a wave of
+// their own selection (prox_select.hip) is as fast or faster from k = 9 on,
+// for fp64 (m = 1000, k = 5: 160 us against 124) and beyond 1024 rows
+// (m = 1500 fp32: 70 us against 64).
+inline bool topk_in_registers(int op, int data, int64_t m, int64_t k) {
+  if (m <= 512) return k <= 15;
+  return data == SDCA_F32 && m <= 1024 && k <= 8 && op != OP_TOPK_CONE_BIASED;
+}
 
 struct ProxLaunch {
   int op;
@@ -75,8 +83,12 @@ hipError_t launch_ent_biased(const ProxLaunch& a);
 hipError_t launch_two_ent(const ProxLaunch& a);
 hipError_t launch_topkent(const ProxLaunch& a);
 hipError_t launch_two(const ProxLaunch& a);
-// Workgroup-per-column kernel over the flagged list (all_columns: every column).
-hipError_t launch_slow(const ProxLaunch& a, bool all_columns);
+// Top-k operators by selection (prox_select.hip), over the flagged list or
+// (all_columns) every column, for the columns select_supported says.
+bool select_supported(const ProxLaunch& a);
+hipError_t launch_select(const ProxLaunch& a, bool all_columns);
+// Every column sorted whole, one workgroup per column.
+hipError_t launch_slow(const ProxLaunch& a);
 // Columns beyond the LDS copy, every column: the sorted-column kernel with
 // each workgroup's column sorted in a slice of scratch (device memory,
 // scratch_bytes; at least one slice of the next power of two above m

@@ -1,0 +1,800 @@
+// Top-k prox columns by selection: the top-k simplex, the top-k cone and
+// their biased forms for the columns the register kernel does not take
+// (topk_in_registers) and for those it defers (the U/M searches).
+//
+// One group of BT threads per column: a wave up to kRegMaxM rows (four
+// independent waves per workgroup), the whole workgroup beyond.  The column
+// is read once into registers.  A cut that certainly lies below every value
+// the thresholds depend on comes from the 64 maxima of 64 disjoint parts of
+// the column (the k + 1 largest of them are k + 1 of its values, so the
+// (k + 1)-th of the maxima is at most its (k + 1)-th largest); the values
+// above the cut, a few more than k + 1 of them, are compacted into LDS,
+// sorted by one wave in its registers and given prefix sums.  The
+// reference's special cases (topk_cone.h:18-55), the knapsack's partition
+// (knapsack_eq.h:25-109) and the U/M searches (topk_cone.h:58-133,
+// topk_cone_biased.h:9-106) are then found on that short sorted list, one
+// rank or one candidate partition per lane.  Sorting the whole column
+// instead (a bitonic network over m values in LDS, then one lane per |U|
+// walking M) took 45 network stages at m = 1000 and 105 at 10,000 for a
+// list of a dozen values that matter.
+//
+// What bounds it: HBM from about 1000 rows on (one read, one write), below
+// that the fixed work per column (two sorts of 64 values, the searches).
+// Measured on MI355X, 40e6 fp32 entries, us per launch, sorting the whole
+// column -> selection:
+//   top-k simplex k = 10:  m = 700 2568 -> 92, 1000 1875 -> 70,
+//                          1500 2261 -> 64, 8000 2523 -> 74, 30000 11841 -> 79
+//   top-k cone k = 5 on margins (U/M searches):  m = 100 12812 -> 653,
+//                          1000 15076 -> 443, 3000 7918 -> 105
+// (one read and one write of them take 52 us at the rate of a large copy
+// kernel).  A column that the list cannot decide (more than kSelectMax values above the cut and no
+// plain knapsack, values that are not finite, ties with zero, a partition
+// that may reach past the list) is sorted whole by the group that holds it
+// (prox_sorted.hpp).
+#include <algorithm>
+#include <climits>
+
+#include "common.hpp"
+#include "prox_impl.hpp"
+#include "prox_launch.hpp"
+#include "prox_sorted.hpp"
+
+namespace sdca_gpu {
+
+namespace {
+
+// Most values of the sorted list (four per lane of a wave).
+constexpr int kSelectMax = 256;
+// Waves per workgroup of the wave-per-column form.
+constexpr int kSelectWaves = 4;
+// Part maxima whose rank gives the cut for a search that may need more than
+// the k + 1 largest: about 64 log(64 / (64 - r)) values lie above the r-th.
+constexpr int kSearchRank = 24;
+constexpr int kSearchRankLast = 56;
+
+// Group-wide synchronisation of a column's LDS.
+template <int BT>
+__device__ inline void select_sync() {
+  if constexpr (BT > 64) __syncthreads();
+  else wave_lds_sync();
+}
+template <int BT>
+__device__ inline int select_lane() {
+  return static_cast<int>(threadIdx.x) & (BT > 64 ? BT - 1 : 63);
+}
+
+// Descending bitonic sort of a wave's 64 * CC values, element l * CC + c in
+// slot c of lane l; each compare-exchange is one median with a bound of +inf
+// (keep the larger) or -inf (keep the smaller), as in group_sort_desc.
+template <int SIZE, int STRIDE, int CC, class D>
+__device__ inline void wave_sort_stage(D (&x)[CC], int lane, D pinf) {
+  constexpr int N = 64 * CC;
+  if constexpr (STRIDE < CC) {
+#pragma unroll
+    for (int c = 0; c < CC; ++c) {
+      if ((c & STRIDE) == 0) {
+        const bool desc = SIZE >= N || (SIZE < CC ? (c & SIZE) == 0 : (lane & (SIZE / CC)) == 0);
+        const D a = x[c], b = x[c + STRIDE];
+        const D bound = desc ? pinf : -pinf;
+        x[c] = max_or_min(a, b, bound);
+        x[c + STRIDE] = max_or_min(a, b, -bound);
+      }
+    }
+  } else {
+    constexpr int L = STRIDE / CC;
+    const bool desc = SIZE >= N || (lane & (SIZE / CC)) == 0;
+    const D bound = (desc == ((lane & L) == 0)) ? pinf : -pinf;
+#pragma unroll
+    for (int c = 0; c < CC; ++c) x[c] = max_or_min(x[c], xor_lane<L, true>(x[c]), bound);
+  }
+  if constexpr (STRIDE > 1) wave_sort_stage<SIZE, STRIDE / 2, CC>(x, lane, pinf);
+}
+template <int SIZE, int CC, class D>
+__device__ inline void wave_sort_from(D (&x)[CC], int lane, D pinf) {
+  wave_sort_stage<SIZE, SIZE / 2, CC>(x, lane, pinf);
+  if constexpr (SIZE < 64 * CC) wave_sort_from<2 * SIZE, CC>(x, lane, pinf);
+}
+template <int CC, class D>
+__device__ inline void wave_sort_desc(D (&x)[CC]) {
+  wave_sort_from<2, CC>(x, static_cast<int>(threadIdx.x) & 63, net_inf(D(0)));
+}
+
+// Exclusive prefix sum over the wave (as wave_exclusive_scan_dpp).
+__device__ inline double wave_exclusive_scan(double x) {
+  double incl = x;
+  incl = dpp_add<0x111, 0xF, true>(incl);   // row_shr:1
+  incl = dpp_add<0x112, 0xF, true>(incl);   // row_shr:2
+  incl = dpp_add<0x114, 0xF, true>(incl);   // row_shr:4
+  incl = dpp_add<0x118, 0xF, true>(incl);   // row_shr:8
+  incl = dpp_add<0x142, 0xA, false>(incl);  // row_bcast:15
+  incl = dpp_add<0x143, 0xC, false>(incl);  // row_bcast:31
+  return incl - x;
+}
+
+// The list's cnt <= 64 CC values sorted in place, and ps[i] = the sum of its
+// first i values in double, i <= cnt.  One wave.
+template <int CC, class D>
+__device__ inline void list_sort(D* list, double* ps, int cnt) {
+  const int lane = static_cast<int>(threadIdx.x) & 63;
+  D x[CC];
+#pragma unroll
+  for (int c = 0; c < CC; ++c) {
+    const int i = lane * CC + c;
+    x[c] = (i < cnt) ? list[i] : -num<D>::inf();
+  }
+  wave_sort_desc<CC>(x);
+  double tot = 0;
+#pragma unroll
+  for (int c = 0; c < CC; ++c) tot += (lane * CC + c < cnt) ? static_cast<double>(x[c]) : 0.0;
+  double run = wave_exclusive_scan(tot);
+  wave_lds_sync();
+#pragma unroll
+  for (int c = 0; c < CC; ++c) {
+    const int i = lane * CC + c;
+    if (i < cnt) {
+      list[i] = x[c];
+      ps[i] = run;
+      run += static_cast<double>(x[c]);
+      if (i == cnt - 1) ps[cnt] = run;
+    }
+  }
+  wave_lds_sync();
+}
+
+// The record of a column, or why there is none yet.
+enum { SEL_DONE = 0, SEL_FIX = 1, SEL_U0 = 2, SEL_WIDER = 3, SEL_SLOW = 4 };
+template <class R>
+struct SelectRecord {
+  R t, hi;
+  int state, branch, n_hi, n_mid;
+};
+
+// The partition of the knapsack sum_i clamp(a_i - t, 0, hi) = rhs on the
+// sorted list (every value above t is in it): rank r is above t where
+// f(a_r) < rhs and at hi where f(a_r - hi) <= rhs, one rank per lane, f from
+// the prefix sums and a binary search for the ranks at hi (or inside) at
+// that point.  The same eps as the fixing's (topk_sorted_root).  The
+// threshold is formed from the direct sum over the free ranks; with none
+// free any t of [a_u, a_(u-1) - hi] is the same projection and the record
+// takes the middle.
+template <class D, class R>
+__device__ inline void list_knapsack(const D* list, const double* ps, int cnt, int m, D cut, R hi_r,
+                                     R rhs_r, R& t_out, int& u_out, int& e_out) {
+  const int lane = static_cast<int>(threadIdx.x) & 63;
+  const double hi = static_cast<double>(hi_r), rhs = static_cast<double>(rhs_r);
+  const double eps = static_cast<double>(num<R>::eps() * dmax(R(1), fabs(rhs_r)));
+  int e = 0, u = 0;
+  for (int base = 0; base < cnt; base += 64) {
+    const int r = base + lane;
+    bool above = false, at_hi = false;
+    if (r < cnt) {
+      const double a = static_cast<double>(list[r]);
+      int b = 0, w = r;
+      while (b < w) {  // ranks above a + hi
+        const int mid = (b + w) >> 1;
+        if (static_cast<double>(list[mid]) > a + hi) b = mid + 1;
+        else w = mid;
+      }
+      above = ps[r] - ps[w] - static_cast<double>(r - w) * a + static_cast<double>(w) * hi < rhs - eps;
+      int z = cnt;
+      b = r + 1;
+      while (b < z) {  // ranks above a - hi
+        const int mid = (b + z) >> 1;
+        if (static_cast<double>(list[mid]) > a - hi) b = mid + 1;
+        else z = mid;
+      }
+      at_hi = static_cast<double>(r + 1) * hi + (ps[z] - ps[r + 1]) -
+                  static_cast<double>(z - r - 1) * (a - hi) <= rhs + eps;
+    }
+    e += __popcll(__ballot(above));
+    u += __popcll(__ballot(at_hi));
+    if (base + 64 > e && base + 64 > u) break;  // no later rank is above t
+  }
+  if (u > e) u = e;
+  if (e > u) {
+    double s = 0;
+    for (int i = u + lane; i < e; i += 64) s += static_cast<double>(list[i]);
+    s = wave_total(s);
+    t_out = static_cast<R>((s + static_cast<double>(u) * hi - rhs) / static_cast<double>(e - u));
+  } else {
+    const double top = (u > 0 ? static_cast<double>(list[u - 1]) : static_cast<double>(list[0])) - hi;
+    double low = top;
+    if (u < cnt) low = static_cast<double>(list[u]);
+    else if (u < m) low = static_cast<double>(cut);
+    t_out = static_cast<R>(0.5 * (low + top));
+  }
+  u_out = u;
+  e_out = e;
+}
+
+// topk_cone_search (topk_cone.h:58-133) and its biased form
+// (topk_cone_biased.h:9-106) on the sorted list, from |U| = u_first on: for
+// each |U| = u the candidate ends e of M = ranks [u, e) are tried by the
+// lanes, the smallest accepted e of the smallest u wins, as in the
+// reference's order.  The list holds the column's cnt largest values, the
+// others are at most `cut`.  Where a search for some u may continue past
+// the list (no end accepted, and t not certainly above every M that would;
+// the bound of cone_biased_regs) the result is SEL_WIDER.
+template <class D, class R>
+__device__ inline SelectRecord<R> list_cone(const D* list, const double* ps, int cnt, int m, D cut,
+                                            int k, R rho, int u_first) {
+  const int lane = static_cast<int>(threadIdx.x) & 63;
+  const R eps = R(16) * num<R>::eps();
+  const R K = static_cast<R>(k);
+  SelectRecord<R> rec;
+  rec.state = SEL_DONE;
+  rec.branch = SDCA_BRANCH_SCAN;
+  for (int u = u_first; u <= k; ++u) {
+    const R k_u = static_cast<R>(k - u);
+    const R nu = rho * K * K + static_cast<R>(u);
+    const double pu = ps[u];
+    const R sum_u = static_cast<R>(pu);
+    const R min_u = u > 0 ? static_cast<R>(list[u - 1]) : num<R>::inf();
+    const R first = u < cnt ? static_cast<R>(list[u]) : -num<R>::inf();
+    for (int e0 = u;; e0 += 64) {
+      const int e = e0 + lane;
+      const bool in = e <= cnt;
+      const int ei = in ? e : cnt;
+      const R n_m = static_cast<R>(ei - u);
+      const R sum_m = static_cast<R>(ps[ei] - pu);
+      const R den = k_u * k_u + n_m * nu;
+      const R t = (nu * sum_m - k_u * sum_u) / den;
+      const R hi = (n_m * sum_u + k_u * sum_m) / den;
+      const R max_m = ei > u ? first : -num<R>::inf();
+      const R min_m = ei > u ? static_cast<R>(list[ei - 1]) : num<R>::inf();
+      const R tt = hi + t;
+      const bool pass = in && max_m - eps <= tt && tt <= min_u + eps && t <= min_m + eps;
+      const R next = ei < cnt ? static_cast<R>(list[ei]) : static_cast<R>(cut);
+      const bool take = pass && (ei == m || next - eps <= t);
+      const unsigned long long taken = __ballot(take);
+      if (taken) {
+        const int l = __ffsll(taken) - 1;
+        rec.t = read_lane(t, __builtin_amdgcn_readfirstlane(l));
+        rec.hi = read_lane(hi, __builtin_amdgcn_readfirstlane(l));
+        rec.n_hi = u;
+        rec.n_mid = e0 + l - u;
+        return rec;
+      }
+      // Nothing accepted up to e: where t is certainly above every later
+      // min(M) (the bound above, next the largest value still to come), the
+      // search for this u is over.
+      const R tol = R(2) * eps + R(8) * num<R>::eps() * dmax(fabs(t), fabs(next));
+      const bool ends = den * (t - next) > tol * (den + static_cast<R>(m - ei) * nu);
+      if (e0 + 64 > cnt) {
+        if (cnt < m && __ballot(in && e == cnt && (pass || !ends))) {
+          rec.state = SEL_WIDER;
+          return rec;
+        }
+        break;
+      }
+      if (__ballot(in && ends)) break;
+    }
+  }
+  rec.t = rec.hi = R(0);
+  rec.branch = SDCA_BRANCH_DEFAULT;
+  rec.n_hi = rec.n_mid = 0;
+  return rec;
+}
+
+// The record from the sorted list (list_sort): thresholds_topk_cone,
+// thresholds_topk_simplex and the biased forms (topk_cone.h:18-157,
+// topk_simplex.h:39-68, topk_simplex_biased.h:40-71,
+// topk_cone_biased.h:98-113).  complete: every value above the knapsack's
+// threshold is in the list (otherwise the special cases only, and SEL_FIX).
+template <class D, class R>
+__device__ inline SelectRecord<R> list_record(const D* list, const double* ps, int cnt, int m, D cut,
+                                              const ProxParamsT<R>& pp, bool complete) {
+  const int k = pp.k;
+  const R K = static_cast<R>(k);
+  const R rho = pp.rho, rhs = pp.rhs;
+  const R eps16 = R(16) * num<R>::eps();
+  const bool cone = pp.op == OP_TOPK_CONE || pp.op == OP_TOPK_CONE_BIASED;
+  SelectRecord<R> rec;
+  rec.state = SEL_DONE;
+  rec.t = rec.hi = R(0);
+  rec.branch = SDCA_BRANCH_ZERO;
+  rec.n_hi = rec.n_mid = 0;
+  const R sum_k = static_cast<R>(ps[k]);
+  if (sum_k <= eps16) return rec;
+  const R hi_c = sum_k / (K + rho * K * K);
+  const R t_c = static_cast<R>(list[k - 1]) - hi_c;
+  const bool constant = k == m || t_c >= static_cast<R>(list[k < cnt ? k : k - 1]) - eps16;
+  const R eps = num<R>::eps() * dmax(R(1), fabs(rhs));
+  if (constant && (cone || !(K * hi_c > rhs + eps))) {
+    rec.t = t_c;
+    rec.hi = hi_c;
+    rec.branch = SDCA_BRANCH_CONSTANT;
+    rec.n_hi = k;
+    return rec;
+  }
+  if (!cone) {
+    if (!complete) {
+      rec.state = SEL_FIX;
+      return rec;
+    }
+    int u, e;
+    list_knapsack<D, R>(list, ps, cnt, m, cut, pp.rhs_k, rhs, rec.t, u, e);
+    bool lt = false;
+    if (!constant) {
+      if (u == 0) {
+        lt = rec.t < rho * rhs - eps;
+      } else {
+        const R num_u = static_cast<R>(u);
+        lt = K * (static_cast<R>(ps[u]) + (K - num_u) * rec.t) < rhs * (num_u + rho * K * K) - eps;
+      }
+    }
+    if (!lt) {
+      rec.hi = pp.rhs_k;
+      rec.branch = SDCA_BRANCH_KNAPSACK;
+      rec.n_hi = u;
+      rec.n_mid = e - u;
+      return rec;
+    }
+  }
+  // Without the bias the search's U = 0 partition is every value above 16
+  // eps: its sum needs the whole column.
+  if (rho == R(0)) {
+    rec.state = SEL_U0;
+    return rec;
+  }
+  return list_cone<D, R>(list, ps, cnt, m, cut, k, rho, 0);
+}
+
+template <class D, class R, int BT, int C>
+__global__ void __launch_bounds__(BT > 64 ? BT : 64 * kSelectWaves)
+prox_select_kernel(const D* __restrict__ in, D* __restrict__ out, int64_t m64, int64_t n,
+                   ProxParamsT<R> pp, sdca_thresholds* __restrict__ thr, int* __restrict__ slow,
+                   int all_columns, int pow2, int group_bytes, int vec,
+                   sdca_prox_sets* __restrict__ sets) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  __shared__ SelectRecord<R> sh_rec[BT > 64 ? 1 : kSelectWaves];
+  __shared__ D sh_cut[BT > 64 ? 1 : kSelectWaves];
+  __shared__ int sh_cnt[2];  // the workgroup's compaction counter, two in turn
+  constexpr int NG = BT > 64 ? 1 : kSelectWaves;  // groups per workgroup
+  const int grp = BT > 64 ? 0 : static_cast<int>(threadIdx.x) >> 6;
+  const int lane = static_cast<int>(threadIdx.x) & 63;
+  const bool lead = BT == 64 || threadIdx.x < 64;  // the wave that solves
+  // The group's LDS: the sorted list and its prefix sums (and the waves'
+  // part maxima), or the whole column where it is sorted.
+  unsigned char* const base = smem_raw + static_cast<size_t>(grp) * group_bytes;
+  double* const ps = reinterpret_cast<double*>(base);
+  D* const list = reinterpret_cast<D*>(base + 8 * (kSelectMax + 2));
+  D* const parts = list + kSelectMax;
+  D* const whole = reinterpret_cast<D*>(base);
+  SelectRecord<R>& rec_lds = sh_rec[grp];
+  const int m = static_cast<int>(m64);
+  const int k = pp.k;
+  const bool cone = pp.op == OP_TOPK_CONE || pp.op == OP_TOPK_CONE_BIASED;
+  const int64_t count = all_columns ? n : static_cast<int64_t>(slow[0]);
+  for (int64_t w = static_cast<int64_t>(blockIdx.x) * NG + grp; w < count;
+       w += static_cast<int64_t>(gridDim.x) * NG) {
+    const int64_t j = all_columns ? w : static_cast<int64_t>(slow[2 + w]);
+    const D* const col = in + j * m64;
+    // (opaque per column: the slots' indices and addresses, hoisted out of
+    // this loop, would hold three registers per slot)
+    int tid = select_lane<BT>();
+    asm("" : "+v"(tid));
+    D v[C];
+    bool finite = true;
+    if (vec) {
+      constexpr int E = 16 / static_cast<int>(sizeof(D));
+      typedef D word __attribute__((ext_vector_type(E)));
+#pragma unroll
+      for (int q = 0; q < C / E; ++q) {
+        const int i = (q * BT + tid) * E;
+        const bool ok = i < m;
+        const word x = *reinterpret_cast<const word*>(col + (ok ? i : 0));
+#pragma unroll
+        for (int l = 0; l < E; ++l) {
+          finite = finite && fabs(x[l]) < num<D>::inf();
+          v[q * E + l] = ok ? x[l] : -num<D>::inf();
+        }
+      }
+    } else {
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        const int i = c * BT + tid;
+        const D x = col[i < m ? i : 0];
+        finite = finite && fabs(x) < num<D>::inf();
+        v[c] = i < m ? x : -num<D>::inf();
+      }
+    }
+    // The maxima of the column's 64 parts (part l: lane l of every wave),
+    // descending over the solving wave's lanes.
+    D part = v[0];
+#pragma unroll
+    for (int c = 1; c < C; ++c) part = (v[c] > part) ? v[c] : part;
+    if (!finite) part = num<D>::inf();  // seen below: the column goes to the sort
+    if constexpr (BT > 64) {
+      parts[threadIdx.x] = part;
+      if (threadIdx.x == 0) sh_cnt[0] = sh_cnt[1] = 0;
+      __syncthreads();
+      if (lead) {
+#pragma unroll
+        for (int i = 1; i < BT / 64; ++i) {
+          const D y = parts[64 * i + lane];
+          part = (y > part) ? y : part;
+        }
+      }
+    }
+    if (lead) {
+      D one[1] = {part};
+      wave_sort_desc<1>(one);
+      part = one[0];
+    }
+    SelectRecord<R> rec;
+    rec.state = SEL_WIDER;
+    rec.t = rec.hi = R(0);
+    rec.branch = rec.n_hi = rec.n_mid = 0;
+    D cut = -num<D>::inf();
+    // At most three lists: the cut for the operator's usual case, a higher
+    // one if that list is too long, a lower one if a search needs more.
+    for (int attempt = 0; attempt < 3; ++attempt) {
+      if (lead) {
+        const D top = read_lane(part, 0);
+        // (a short column is its own list: -inf is the padding)
+        D c = -num<D>::max_finite();
+        if (m > kSelectMax) {
+          // the k + 1 largest, and for the knapsack every value above
+          // a_(k) - hi; a search's list from further down
+          c = read_lane(part, (cone && attempt == 0 && k < kSearchRank) ? kSearchRank : k);
+          if (!cone && attempt != 1) {
+            const R b = static_cast<R>(c);
+            const D lower = static_cast<D>(b - pp.rhs_k -
+                                           (fabs(b) + pp.rhs_k) * (R(16) * num<R>::eps()));
+            c = lower < c ? lower : c;
+          }
+          if (attempt == 2) {
+            const D last = read_lane(part, kSearchRankLast);
+            c = last < c ? last : c;
+          }
+        }
+        if (!(top < num<D>::inf())) c = num<D>::quiet_nan();
+        cut = c;
+        if constexpr (BT > 64) {
+          if (threadIdx.x == 0) sh_cut[0] = c;
+        }
+      }
+      if constexpr (BT > 64) {
+        __syncthreads();
+        cut = sh_cut[0];
+      }
+      if (!(cut == cut)) {
+        rec.state = SEL_SLOW;
+        break;
+      }
+      // The values at or above the cut, in any order.
+      int cnt = 0;
+      if constexpr (BT == 64) {
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+          const bool pr = v[c] >= cut;
+          const unsigned long long mask = __ballot(pr);
+          if (mask) {
+            const int at = cnt + static_cast<int>(__builtin_amdgcn_mbcnt_hi(
+                static_cast<unsigned>(mask >> 32),
+                __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(mask), 0)));
+            if (pr && at < kSelectMax) list[at] = v[c];
+            cnt += __popcll(mask);
+          }
+        }
+        wave_lds_sync();
+      } else {
+        int mine = 0;
+#pragma unroll
+        for (int c = 0; c < C; ++c) mine += __popcll(__ballot(v[c] >= cut));
+        int at0 = 0;
+        if (mine > 0) {
+          if (lane == 0) at0 = atomicAdd(&sh_cnt[attempt & 1], mine);
+          at0 = __builtin_amdgcn_readfirstlane(at0);
+#pragma unroll
+          for (int c = 0; c < C; ++c) {
+            const bool pr = v[c] >= cut;
+            const unsigned long long mask = __ballot(pr);
+            if (mask) {
+              const int at = at0 + static_cast<int>(__builtin_amdgcn_mbcnt_hi(
+                  static_cast<unsigned>(mask >> 32),
+                  __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(mask), 0)));
+              if (pr && at < kSelectMax) list[at] = v[c];
+              at0 += __popcll(mask);
+            }
+          }
+        }
+        __syncthreads();
+        cnt = sh_cnt[attempt & 1];
+        if (threadIdx.x == 0) sh_cnt[(attempt & 1) ^ 1] = 0;
+      }
+      if (cnt > kSelectMax) {
+        if (attempt == 0) continue;  // the higher cut of attempt 1
+        rec.state = SEL_SLOW;
+        break;
+      }
+      if (lead) {
+        if (cnt <= 64) list_sort<1>(list, ps, cnt);
+        else if (cnt <= 128) list_sort<2>(list, ps, cnt);
+        else list_sort<4>(list, ps, cnt);
+        rec = list_record<D, R>(list, ps, cnt, m, cut, pp, cone || attempt != 1);
+      }
+      if constexpr (BT > 64) {
+        if (threadIdx.x == 0) rec_lds = rec;
+        __syncthreads();
+        rec = rec_lds;
+      }
+      if (rec.state == SEL_U0) {
+        // topk_cone_search with U empty: t = 0, M = {x > 16 eps}, then the
+        // n_z values within 16 eps of zero one by one.  (This pass
+        // and the fixing below read the column again, from the L2: unrolled
+        // over the slots they set the kernel's register peak.)
+        const R eps16 = R(16) * num<R>::eps();
+        R s_p = 0;
+        int n_p = 0, n_z = 0;
+#pragma unroll 4
+        for (int i = tid; i < m; i += BT) {
+          const R x = static_cast<R>(col[i]);
+          const bool pos = x > eps16;
+          s_p += pos ? x : R(0);
+          n_p += pos ? 1 : 0;
+          n_z += (!pos && x >= -eps16) ? 1 : 0;
+        }
+        group_sums<BT>(s_p, n_p, n_z);
+        const R K = static_cast<R>(k);
+        const R hi = (K * s_p) / (K * K);
+        const R largest = n_p > 0 ? static_cast<R>(list[0]) : -num<R>::inf();
+        rec.state = SEL_DONE;
+        rec.t = R(0);
+        rec.hi = hi;
+        rec.branch = SDCA_BRANCH_SCAN;
+        rec.n_hi = 0;
+        rec.n_mid = n_p;
+        if (largest - eps16 <= hi) {
+          // accepted at the first end the reference tries
+        } else if (largest - eps16 <= hi + static_cast<R>(n_z) * eps16) {
+          rec.state = SEL_SLOW;  // the values near zero may decide
+        } else {
+          if (lead) rec = list_cone<D, R>(list, ps, cnt, m, cut, k, R(0), 1);
+          if constexpr (BT > 64) {
+            __syncthreads();
+            if (threadIdx.x == 0) rec_lds = rec;
+            __syncthreads();
+            rec = rec_lds;
+          }
+        }
+      }
+      if (rec.state == SEL_FIX) {
+        // More candidates than the list holds: variable fixing over the
+        // slots, the free set as the value interval (lc, hc].
+        const R hi = pp.rhs_k, rhs = pp.rhs;
+        const R eps = num<R>::eps() * dmax(R(1), fabs(rhs));
+        const R kth = static_cast<R>(list[k - 1]);
+        const R slack = (fabs(kth) + hi) * (R(16) * num<R>::eps());
+        R lc = kth - hi - slack, hc = kth + hi + slack;
+        R s_f = 0, s_u = 0;
+        int n_f = 0, n_u = 0;
+#pragma unroll 4
+        for (int i = tid; i < m; i += BT) {
+          const R x = static_cast<R>(col[i]);
+          const bool f = x > lc && x <= hc;
+          s_f += f ? x : R(0);
+          n_f += f ? 1 : 0;
+          s_u += x > hc ? x : R(0);
+          n_u += x > hc ? 1 : 0;
+        }
+        group_sums<BT>(s_f, s_u, n_f, n_u);
+        R t = div_near(s_f + static_cast<R>(n_u) * hi - rhs, static_cast<R>(n_f));
+        for (int iter = 0; iter <= m; ++iter) {
+          const R c_hi = hi + t;
+          R s_lo = 0, s_hi = 0;
+          int n_lo = 0, n_hi = 0;
+#pragma unroll 4
+          for (int i = tid; i < m; i += BT) {
+            const R x = static_cast<R>(col[i]);
+            const bool f = x > lc && x <= hc;
+            s_lo += (f && x <= t) ? x : R(0);
+            n_lo += (f && x <= t) ? 1 : 0;
+            s_hi += (f && x > c_hi) ? x : R(0);
+            n_hi += (f && x > c_hi) ? 1 : 0;
+          }
+          group_sums<BT>(s_lo, s_hi, n_lo, n_hi);
+          const R infeas = s_hi + s_lo - static_cast<R>(n_hi) * hi - static_cast<R>(n_hi + n_lo) * t;
+          const bool fix_hi = n_hi > 0 && infeas > eps;
+          const bool fix_lo = !fix_hi && n_lo > 0 && infeas < -eps;
+          if (fix_hi || (!fix_lo && n_hi > 0)) {
+            hc = c_hi;
+            n_u += n_hi;
+            s_u += s_hi;
+            n_f -= n_hi;
+          }
+          if (fix_lo || (!fix_hi && n_lo > 0)) {
+            lc = t;
+            n_f -= n_lo;
+          }
+          if (n_f <= 0) break;
+          s_f = 0;
+#pragma unroll 4
+          for (int i = tid; i < m; i += BT) {
+            const R x = static_cast<R>(col[i]);
+            s_f += (x > lc && x <= hc) ? x : R(0);
+          }
+          s_f = group_sum<BT>(s_f);
+          t = div_near(s_f + static_cast<R>(n_u) * hi - rhs, static_cast<R>(n_f));
+          if (!fix_hi && !fix_lo) break;
+        }
+        bool lt;
+        const R K = static_cast<R>(k), num_u = static_cast<R>(n_u);
+        if (n_u == 0) lt = t < pp.rho * rhs - eps;
+        else lt = K * (s_u + (K - num_u) * t) < rhs * (num_u + pp.rho * K * K) - eps;
+        const R sum_k = static_cast<R>(ps[k]);
+        const bool constant = static_cast<R>(list[k - 1]) - sum_k / (K + pp.rho * K * K) >=
+                              static_cast<R>(list[k]) - R(16) * num<R>::eps();
+        rec.state = (lt && !constant) ? SEL_SLOW : SEL_DONE;
+        rec.t = t;
+        rec.hi = hi;
+        rec.branch = SDCA_BRANCH_KNAPSACK;
+        rec.n_hi = n_u;
+        rec.n_mid = n_f;
+        break;
+      }
+      if (rec.state != SEL_WIDER) break;
+      // One wider list, where this was the usual one.
+      if (m <= kSelectMax || attempt != 0) {
+        rec.state = SEL_SLOW;
+        break;
+      }
+      if constexpr (BT > 64) __syncthreads();
+      else wave_lds_sync();
+      attempt = 1;  // the lower cut next
+      if constexpr (BT > 64) {
+        if (threadIdx.x == 0) sh_cnt[0] = 0;
+        __syncthreads();
+      }
+    }
+    R lo = R(0);
+    if (rec.state != SEL_DONE) {
+      // The whole column sorted in the group's LDS.
+      select_sync<BT>();
+      for (int i = tid; i < pow2; i += BT) whole[i] = (i < m) ? col[i] : -num<D>::inf();
+      select_sync<BT>();
+      for (int size = 2; size <= pow2; size <<= 1) {
+        for (int stride = size >> 1; stride > 0; stride >>= 1) {
+          for (int i = tid; i < pow2; i += BT) {
+            const int partner = i ^ stride;
+            if (partner > i) {
+              const bool desc = (i & size) == 0;
+              const D a = whole[i], b = whole[partner];
+              if (desc ? (a < b) : (b < a)) {
+                whole[i] = b;
+                whole[partner] = a;
+              }
+            }
+          }
+          select_sync<BT>();
+        }
+      }
+      if (lead)
+        thresholds_sorted<D, R>(whole, m, pp.op, pp.lo, pp.hi, pp.rhs, pp.rho, k, rec.t, lo, rec.hi,
+                                rec.branch, rec.n_hi, rec.n_mid);
+      if constexpr (BT > 64) {
+        if (threadIdx.x == 0) rec_lds = rec;
+        __syncthreads();
+        rec = rec_lds;
+      }
+      lo = R(0);
+    }
+    if (tid == 0) {
+      if (thr)
+        thr[j] = sdca_thresholds{static_cast<double>(rec.t), static_cast<double>(lo),
+                                 static_cast<double>(rec.hi)};
+      if (sets) sets[j] = sdca_prox_sets{rec.n_hi, rec.n_mid, rec.branch, 0};
+    }
+    const D t = static_cast<D>(rec.t), dlo = D(0), dhi = static_cast<D>(rec.hi);
+    asm("" : "+v"(tid));
+    D* const dst = out + j * m64;
+    if (vec) {
+      constexpr int E = 16 / static_cast<int>(sizeof(D));
+      typedef D word __attribute__((ext_vector_type(E)));
+#pragma unroll
+      for (int q = 0; q < C / E; ++q) {
+        const int i = (q * BT + tid) * E;
+        word y;
+#pragma unroll
+        for (int l = 0; l < E; ++l) y[l] = clamp_ref(v[q * E + l] - t, dlo, dhi);
+        if (i < m) __builtin_nontemporal_store(y, reinterpret_cast<word*>(dst + i));
+      }
+    } else {
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        const int i = c * BT + tid;
+        if (i < m) dst[i] = clamp_ref(v[c] - t, dlo, dhi);
+      }
+    }
+    select_sync<BT>();  // the column's LDS before the next one's
+  }
+  // List mode: the list's counters [count, done] must be zero for the next
+  // call on the stream.  With an empty list they already are; otherwise the
+  // workgroups that took columns count themselves out and the last of them
+  // zeroes both (each has read the count before it increments done).
+  if (!all_columns) {
+    const int64_t groups = (count + NG - 1) / NG;
+    const int64_t workers = groups < static_cast<int64_t>(gridDim.x) ? groups : gridDim.x;
+    if (NG > 1) __syncthreads();
+    if (static_cast<int64_t>(blockIdx.x) < workers && threadIdx.x == 0) {
+      __threadfence();
+      if (atomicAdd(slow + 1, 1) == static_cast<int>(workers) - 1) {
+        atomicExch(slow, 0);
+        atomicExch(slow + 1, 0);
+      }
+    }
+  }
+}
+
+template <class D, class R, int BT, int C>
+hipError_t select_one(const ProxLaunch& a, bool all_columns) {
+  ProxParamsT<R> pp;
+  pp.lo = static_cast<R>(a.lo);
+  pp.hi = static_cast<R>(a.hi);
+  pp.rhs = static_cast<R>(a.rhs);
+  const bool biased = a.op == OP_TOPK_SIMPLEX_BIASED || a.op == OP_TOPK_CONE_BIASED;
+  pp.rho = biased ? static_cast<R>(a.rho) : R(0);
+  pp.k = static_cast<int>(a.k);
+  pp.rhs_k = pp.rhs / static_cast<R>(a.k);
+  pp.op = a.op;
+  pp.p = static_cast<int>(a.p);
+  if (a.m > static_cast<int64_t>(BT) * C) return hipErrorInvalidValue;
+  int pow2 = 1;
+  while (pow2 < a.m) pow2 <<= 1;
+  constexpr int NG = BT > 64 ? 1 : kSelectWaves;
+  constexpr int E = 16 / static_cast<int>(sizeof(D));
+  const int64_t list_bytes = 8 * (kSelectMax + 2) +
+                             (kSelectMax + (BT > 64 ? BT : 0)) * static_cast<int64_t>(sizeof(D));
+  const int64_t sort_bytes = static_cast<int64_t>(pow2) * static_cast<int64_t>(sizeof(D));
+  const int64_t group_bytes = (std::max(list_bytes, sort_bytes) + 15) / 16 * 16;
+  const int vec = a.m % E == 0 &&
+                  ((reinterpret_cast<uintptr_t>(a.in) | reinterpret_cast<uintptr_t>(a.out)) & 15) == 0;
+  // List mode: the list is usually empty or a small fraction of the n
+  // columns; the grid grows with the batch (256 to 1024 workgroups), so that
+  // a long list finds four waves on every SIMD while an empty one costs
+  // little to launch.
+  const int64_t groups = (a.n + NG - 1) / NG;
+  const int64_t work = a.n * a.m / 16384;
+  const int64_t cap = all_columns ? (int64_t(1) << 30)
+                                  : std::min<int64_t>(1024, std::max<int64_t>(256, work));
+  const int64_t grid = std::max<int64_t>(1, std::min(groups, cap));
+  hipLaunchKernelGGL((prox_select_kernel<D, R, BT, C>), dim3(static_cast<unsigned>(grid)),
+                     dim3(BT > 64 ? BT : 64 * NG), static_cast<size_t>(group_bytes * NG), a.stream,
+                     static_cast<const D*>(a.in), static_cast<D*>(a.out), a.m, a.n, pp, a.thr,
+                     a.slow, all_columns ? 1 : 0, pow2, static_cast<int>(group_bytes), vec, a.sets);
+  return hipGetLastError();
+}
+
+template <class D, class R>
+hipError_t select_by_m(const ProxLaunch& a, bool all_columns) {
+  if (a.m <= 256) return select_one<D, R, 64, 4>(a, all_columns);
+  if (a.m <= 512) return select_one<D, R, 64, 8>(a, all_columns);
+  if (a.m <= 1024) return select_one<D, R, 64, 16>(a, all_columns);
+  if (a.m <= 2048) return select_one<D, R, 64, 32>(a, all_columns);
+  if (a.m <= 4096) return select_one<D, R, 256, 16>(a, all_columns);
+  if (a.m <= 8192) return select_one<D, R, 512, 16>(a, all_columns);
+  if (a.m <= 16384) return select_one<D, R, 1024, 16>(a, all_columns);
+  if constexpr (sizeof(D) == 4) return select_one<D, R, 1024, 32>(a, all_columns);
+  return hipErrorInvalidValue;
+}
+
+}  // namespace
+
+// k + 1 part maxima give the cut, and the last search's rank must lie past
+// them; a column of at most kSelectMax rows is its own list.
+bool select_supported(const ProxLaunch& a) {
+  const bool topk = a.op == OP_TOPK_SIMPLEX || a.op == OP_TOPK_CONE ||
+                    a.op == OP_TOPK_SIMPLEX_BIASED || a.op == OP_TOPK_CONE_BIASED;
+  return topk && a.m <= max_rows(a.data) && (a.m <= kSelectMax || a.k < kSearchRankLast);
+}
+
+hipError_t launch_select(const ProxLaunch& a, bool all_columns) {
+  if (a.data == SDCA_F32 && a.result == SDCA_F32) return select_by_m<float, float>(a, all_columns);
+  if (a.data == SDCA_F32 && a.result == SDCA_F64) return select_by_m<float, double>(a, all_columns);
+  if (a.data == SDCA_F64 && a.result == SDCA_F64) return select_by_m<double, double>(a, all_columns);
+  if (a.data == SDCA_F64 && a.result == SDCA_F32) return select_by_m<double, float>(a, all_columns);
+  return hipErrorInvalidValue;
+}
+
+}  // namespace sdca_gpu

@@ -1,6 +1,6 @@
-// Workgroup-per-column prox kernel: the columns the register kernel defers
-// (topk_cone_search with U non-empty, zero-band ties, k > kTopkMaxK) and the
-// knapsack operators for m beyond the register kernel.
+// Columns sorted whole, one workgroup per column: the top-k operators with k
+// beyond the selection kernel's lists (prox_select.hip), and the operators
+// whose thresholds need the sorted column beyond the LDS.
 //
 // The column is sorted in LDS (bitonic, descending, the order the reference's
 // std::sort(greater) produces), then the first wave runs the reference's
@@ -10,8 +10,9 @@
 // top-k simplex test (topk_simplex.h:9-68) and the O(k m) search
 // topk_cone_search (topk_cone.h:58-133) in the same order - and the
 // workgroup clamps the column from global memory.
-// Columns come from a device list written by the register kernel, so no host
-// round trip is needed; every workgroup exits after the list is drained.
+// Also here: the sort-based two-block simplex (every column, or the columns
+// of a device list written by the register kernel), the two-block simplex
+// and the top-k entropy beyond the LDS, and the elementwise Lambert map.
 #include <algorithm>
 #include <climits>
 
@@ -29,16 +30,13 @@ namespace {
 template <class D, class R, bool GV = false>
 __global__ void __launch_bounds__(256)
 prox_slow_kernel(const D* __restrict__ in, D* __restrict__ out, int64_t m64, int64_t n,
-                 ProxParamsT<R> pp, sdca_thresholds* __restrict__ thr,
-                 int* __restrict__ slow, int all_columns, int pow2,
+                 ProxParamsT<R> pp, sdca_thresholds* __restrict__ thr, int pow2,
                  sdca_prox_sets* __restrict__ sets, D* __restrict__ gscratch) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   D* s = GV ? gscratch + static_cast<int64_t>(blockIdx.x) * pow2 : reinterpret_cast<D*>(smem_raw);
   __shared__ R sh_t, sh_lo, sh_hi;
   const int m = static_cast<int>(m64);
-  const int64_t count = all_columns ? n : static_cast<int64_t>(slow[0]);
-  for (int64_t w = blockIdx.x; w < count; w += gridDim.x) {
-    const int64_t j = all_columns ? w : static_cast<int64_t>(slow[2 + w]);
+  for (int64_t j = blockIdx.x; j < n; j += gridDim.x) {
     const D* col = in + j * m64;
     for (int i = threadIdx.x; i < pow2; i += blockDim.x)
       s[i] = (i < m) ? col[i] : -num<D>::inf();
@@ -85,51 +83,26 @@ prox_slow_kernel(const D* __restrict__ in, D* __restrict__ out, int64_t m64, int
     for (int i = threadIdx.x; i < m; i += blockDim.x) dst[i] = clamp_ref(col[i] - t, lo, hi);
     __syncthreads();
   }
-  // List mode: the list's counters [count, done] must be zero for the next
-  // call on the stream.  With an empty list they already are; otherwise the
-  // min(grid, count) workgroups that took columns count themselves out and
-  // the last of them zeroes both (each has read the count before it
-  // increments done).
-  const int64_t workers = count < static_cast<int64_t>(gridDim.x) ? count : gridDim.x;
-  if (!all_columns && static_cast<int64_t>(blockIdx.x) < workers && threadIdx.x == 0) {
-    __threadfence();
-    if (atomicAdd(slow + 1, 1) == static_cast<int>(workers) - 1) {
-      atomicExch(slow, 0);
-      atomicExch(slow + 1, 0);
-    }
-  }
 }
 
 template <class D, class R>
-hipError_t launch_slow_t(const ProxLaunch& a, bool all_columns) {
+hipError_t launch_slow_t(const ProxLaunch& a) {
   ProxParamsT<R> pp;
   pp.lo = static_cast<R>(a.lo);
   pp.hi = static_cast<R>(a.hi);
   pp.rhs = static_cast<R>(a.rhs);
-  const bool biased = a.op == OP_KNAPSACK_LE_BIASED || a.op == OP_TOPK_SIMPLEX_BIASED ||
-                      a.op == OP_TOPK_CONE_BIASED;
+  const bool biased = a.op == OP_TOPK_SIMPLEX_BIASED || a.op == OP_TOPK_CONE_BIASED;
   pp.rho = biased ? static_cast<R>(a.rho) : R(0);
   pp.k = static_cast<int>(a.k);
   pp.op = a.op;
   pp.p = static_cast<int>(a.p);
   int pow2 = 1;
   while (pow2 < a.m) pow2 <<= 1;
-  // List mode: the list is a small fraction of the n columns and usually
-  // empty; the grid grows with n (about one workgroup per 1024 columns,
-  // 512 to 1024: four per CU), so that a long list finds workgroups on
-  // every CU while an empty one costs little to launch (the launch of 3906
-  // workgroups for an empty C2 list took 0.5 % of the step; 1024 runs the
-  // biased cone's deferred columns as fast).
-  const int64_t cap = all_columns ? 4096 : std::min<int64_t>(1024, std::max<int64_t>(512, a.n / 1024));
-  const int64_t grid = a.n < cap ? a.n : cap;
-  // One wave per workgroup for short columns (the sort's stages then need
-  // no cross-wave barrier and four times as many columns are in flight),
-  // four waves beyond 256 rows.
-  const int threads = pow2 <= 256 ? 64 : 256;
+  const int64_t grid = a.n < 4096 ? a.n : 4096;
   hipLaunchKernelGGL((prox_slow_kernel<D, R>), dim3(static_cast<unsigned>(grid > 0 ? grid : 1)),
-                     dim3(threads), static_cast<size_t>(pow2) * sizeof(D), a.stream,
+                     dim3(256), static_cast<size_t>(pow2) * sizeof(D), a.stream,
                      static_cast<const D*>(a.in), static_cast<D*>(a.out), a.m, a.n, pp,
-                     a.thr, a.slow, all_columns ? 1 : 0, pow2, a.sets, static_cast<D*>(nullptr));
+                     a.thr, pow2, a.sets, static_cast<D*>(nullptr));
   return hipGetLastError();
 }
 
@@ -155,7 +128,7 @@ hipError_t launch_slow_global_t(const ProxLaunch& a, void* scratch, size_t scrat
   if (grid < 1) return hipErrorInvalidValue;
   hipLaunchKernelGGL((prox_slow_kernel<D, R, true>), dim3(static_cast<unsigned>(grid)),
                      dim3(256), 0, a.stream, static_cast<const D*>(a.in), static_cast<D*>(a.out),
-                     a.m, a.n, pp, a.thr, a.slow, 1, static_cast<int>(pow2), a.sets,
+                     a.m, a.n, pp, a.thr, static_cast<int>(pow2), a.sets,
                      static_cast<D*>(scratch));
   return hipGetLastError();
 }
@@ -480,11 +453,11 @@ __global__ void __launch_bounds__(256) lambert_kernel(const D* __restrict__ in, 
 
 }  // namespace
 
-hipError_t launch_slow(const ProxLaunch& a, bool all_columns) {
-  if (a.data == SDCA_F32 && a.result == SDCA_F32) return launch_slow_t<float, float>(a, all_columns);
-  if (a.data == SDCA_F32 && a.result == SDCA_F64) return launch_slow_t<float, double>(a, all_columns);
-  if (a.data == SDCA_F64 && a.result == SDCA_F64) return launch_slow_t<double, double>(a, all_columns);
-  if (a.data == SDCA_F64 && a.result == SDCA_F32) return launch_slow_t<double, float>(a, all_columns);
+hipError_t launch_slow(const ProxLaunch& a) {
+  if (a.data == SDCA_F32 && a.result == SDCA_F32) return launch_slow_t<float, float>(a);
+  if (a.data == SDCA_F32 && a.result == SDCA_F64) return launch_slow_t<float, double>(a);
+  if (a.data == SDCA_F64 && a.result == SDCA_F64) return launch_slow_t<double, double>(a);
+  if (a.data == SDCA_F64 && a.result == SDCA_F32) return launch_slow_t<double, float>(a);
   return hipErrorInvalidValue;
 }
 

@@ -8,6 +8,7 @@ hipError_t launch_topk(const ProxLaunch& a) {
   if (a.op == OP_TOPK_CONE_BIASED) return launch_by_type<FAM_TOPK, 15>(a);
   if (a.k <= 2) return launch_by_type<FAM_TOPK, 2>(a);
   if (a.k <= 5) return launch_by_type<FAM_TOPK, 5>(a);
-  return launch_by_type<FAM_TOPK, 8>(a);
+  if (a.k <= 8) return launch_by_type<FAM_TOPK, 8>(a);
+  return launch_by_type<FAM_TOPK, 15>(a);
 }
 }  // namespace sdca_gpu

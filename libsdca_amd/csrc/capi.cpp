@@ -818,27 +818,35 @@ int sdca_recompute_primal(sdca_dtype data, int64_t d, int64_t m, int64_t n, cons
     pW0 = W0 ? dw0.ptr : nullptr;
     pW = dw.ptr;
   }
-  // W (m x d row-major) = A' (m x n) X (n x d): the score GEMM with both
-  // operands transposed once so that the contraction over n runs along rows.
   void* ws = nullptr;
-  if ((rc = workspace(stream, 3, es * static_cast<size_t>(n) * static_cast<size_t>(m + d), &ws)))
-    return rc;
-  void* At = ws;
-  void* Xt = static_cast<char*>(ws) + es * static_cast<size_t>(n) * static_cast<size_t>(m);
-  SDCA_HIP_TRY(launch_transpose(data, pA, At, n, m, stream), "transpose kernel");
-  SDCA_HIP_TRY(launch_transpose(data, pX, Xt, n, d, stream), "transpose kernel");
-  if (data == SDCA_F32) {
-    void* gws = nullptr;
-    size_t gws_bytes = 0;
-    if ((rc = gemm_workspace(stream, m, d, n, &gws, &gws_bytes))) return rc;
-    SDCA_HIP_TRY(launch_scores_gemm(static_cast<const float*>(At), static_cast<const float*>(Xt),
-                                    static_cast<float*>(pW), m, d, n, stream, gws, gws_bytes),
-                 "GEMM kernel");
-  } else
-    SDCA_HIP_TRY(launch_scores_gemm_f64(static_cast<const double*>(At),
-                                        static_cast<const double*>(Xt), static_cast<double*>(pW),
-                                        m, d, n, stream), "GEMM kernel");
-  if (pW0) SDCA_HIP_TRY(launch_add(data, pW, pW0, d * m, stream), "add kernel");
+  if (!primal_split(data, d, m, n)) {
+    // W (m x d row-major) = A' (m x n) X (n x d): the score GEMM with both
+    // operands transposed once so that the contraction over n runs along
+    // rows.
+    if ((rc = workspace(stream, 3, es * static_cast<size_t>(n) * static_cast<size_t>(m + d), &ws)))
+      return rc;
+    void* At = ws;
+    void* Xt = static_cast<char*>(ws) + es * static_cast<size_t>(n) * static_cast<size_t>(m);
+    SDCA_HIP_TRY(launch_transpose(data, pA, At, n, m, stream), "transpose kernel");
+    SDCA_HIP_TRY(launch_transpose(data, pX, Xt, n, d, stream), "transpose kernel");
+    if (data == SDCA_F32) {
+      void* gws = nullptr;
+      size_t gws_bytes = 0;
+      if ((rc = gemm_workspace(stream, m, d, n, &gws, &gws_bytes))) return rc;
+      SDCA_HIP_TRY(launch_scores_gemm(static_cast<const float*>(At), static_cast<const float*>(Xt),
+                                      static_cast<float*>(pW), m, d, n, stream, gws, gws_bytes),
+                   "GEMM kernel");
+    } else {
+      SDCA_HIP_TRY(launch_scores_gemm_f64(static_cast<const double*>(At),
+                                          static_cast<const double*>(Xt), static_cast<double*>(pW),
+                                          m, d, n, stream), "GEMM kernel");
+    }
+    if (pW0) SDCA_HIP_TRY(launch_add(data, pW, pW0, d * m, stream), "add kernel");
+  } else {
+    if ((rc = workspace(stream, 3, es * static_cast<size_t>(primal_workspace_values(d, m, n)), &ws)))
+      return rc;
+    SDCA_HIP_TRY(launch_primal(data, pX, pA, pW0, pW, ws, d, m, n, stream), "primal GEMM kernels");
+  }
   if (flags & SDCA_HOST_PTR) {
     SDCA_HIP_TRY(hipMemcpyAsync(W, pW, es * d * m, hipMemcpyDeviceToHost, stream), "hipMemcpyAsync(D2H)");
     SDCA_HIP_TRY(hipStreamSynchronize(stream), "hipStreamSynchronize");

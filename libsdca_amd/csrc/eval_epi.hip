@@ -23,8 +23,11 @@
 // fixed order, so the totals are deterministic.  Examples whose top-k
 // simplex needs the reference's full topk_cone_search are listed and
 // finished by the workgroup-per-example kernel at the end of this file.
+#include <algorithm>
+
 #include "eval_launch.hpp"
 #include "prox_impl.hpp"
+#include "prox_sorted.hpp"
 
 namespace sdca_gpu {
 
@@ -851,147 +854,58 @@ eval_multilabel_kernel(const D* __restrict__ S, const D* __restrict__ A,
 
 // ---------------------------------------------------------------------------
 // Deferred smooth top-k hinge examples: the h values of the example are
-// sorted in LDS and one lane runs the reference's thresholds_topk_simplex on
+// sorted in LDS and one wave runs the reference's thresholds_topk_simplex on
 // them (special cases, Kiwiel on contiguous ranges, topk_cone_search), then
 // the loss from the sorted threshold sets.
 // ---------------------------------------------------------------------------
-template <class D, class R>
-__device__ R sorted_sum(const D* s, int b, int e) {
-  double acc = 0, comp = 0;
-  for (int q = b; q < e; ++q) {
-    const double x = static_cast<double>(static_cast<R>(s[q]));
-    const double t = acc + x;
-    comp += (fabs(acc) >= fabs(x)) ? (acc - t) + x : (x - t) + acc;
-    acc = t;
-  }
-  return static_cast<R>(acc + comp);
-}
-
-template <class D, class R>
-__device__ R sorted_dot(const D* s, int b, int e) {
-  double acc = 0;
-  for (int q = b; q < e; ++q) {
-    const double x = static_cast<double>(static_cast<R>(s[q]));
-    acc += x * x;
-  }
-  return static_cast<R>(acc);
-}
-
+// The smooth top-k hinge of the shifted scores s[0, mp) sorted descending,
+// by the 64 lanes of a wave: the thresholds of the top-k simplex
+// (prox_sorted.hpp; their searches and range sums split over the lanes, 138
+// -> 29 us for the deferred examples of a 137-class fp64 set against one
+// lane walking the row), then the loss from the record's sets.
 template <class D, class R>
 __device__ R smooth_topk_sorted(const D* s, int mp, int k, R gamma) {
+  const int lane = static_cast<int>(threadIdx.x) & 63;
   const R K = static_cast<R>(k);
-  const R eps16 = R(16) * num<R>::eps();
-  const R sum_k = sorted_sum<D, R>(s, 0, k);
-  if (sum_k <= eps16) return R(0);
-  const R hi_c = sum_k / K;
-  const R t_c = static_cast<R>(s[k - 1]) - hi_c;
-  const bool constant = (k == mp) || (t_c >= static_cast<R>(s[k]) - eps16);
-  const R eps = num<R>::eps() * dmax(R(1), fabs(gamma));
-  if (constant && !(K * hi_c > gamma + eps)) return hi_c * sum_k - R(0.5) * hi_c * hi_c * K;
-  // Kiwiel on the sorted values: U = [0, f), M = [f, l), L = [l, mp)
-  const R hi = gamma / K;
-  int mc = mp, f = 0, l = mp;
-  R t = (sorted_sum<D, R>(s, 0, mp) - gamma) / static_cast<R>(mp);
-  for (int iter = 0; iter <= mp; ++iter) {
-    const R c_lo = t, c_hi = hi + t;
-    int p_lo = f;
-    while (p_lo < l && static_cast<R>(s[p_lo]) > c_lo) ++p_lo;
-    int p_hi = f;
-    while (p_hi < p_lo && static_cast<R>(s[p_hi]) > c_hi) ++p_hi;
-    const R s_lo = sorted_sum<D, R>(s, p_lo, l);
-    const int n_lo = l - p_lo;
-    const R s_hi = sorted_sum<D, R>(s, f, p_hi);
-    const int n_hi = p_hi - f;
-    const R sh = static_cast<R>(n_hi) * hi;
-    const R infeas = s_hi + s_lo - sh - static_cast<R>(n_hi + n_lo) * t;
-    R next;
-    if (n_hi > 0 && infeas > eps) {
-      f = p_hi;
-      next = static_cast<R>(mc) * t - s_hi + sh;
-      mc -= n_hi;
-    } else if (n_lo > 0 && infeas < -eps) {
-      l = p_lo;
-      next = static_cast<R>(mc) * t - s_lo;
-      mc -= n_lo;
-    } else {
-      f = p_hi;
-      l = p_lo;
-      break;
-    }
-    if (mc > 0) t = next / static_cast<R>(mc);
-    else break;
+  R t, lo, hi;
+  int branch, f, n_mid;
+  thresholds_sorted<D, R>(s, mp, OP_TOPK_SIMPLEX, R(0), gamma, gamma, R(0), k, t, lo, hi, branch, f,
+                          n_mid);
+  if (branch == SDCA_BRANCH_ZERO || branch == SDCA_BRANCH_DEFAULT) return R(0);
+  if (branch == SDCA_BRANCH_CONSTANT) {
+    const R sum_k = sum_range<R>(s, 0, k);
+    return hi * sum_k - R(0.5) * hi * hi * K;
   }
-  bool lt = false;
-  if (!constant) {
-    if (f == 0) {
-      lt = t < -eps;
-    } else {
-      const R num_u = static_cast<R>(f);
-      lt = K * (sorted_sum<D, R>(s, 0, f) + (K - num_u) * t) < gamma * num_u - eps;
-    }
-  }
-  R th = hi;
-  if (lt) {
-    // topk_cone_search (topk_cone.h:58-133) on the sorted values
-    R k_u = K, min_u = num<R>::inf(), num_u = 0, sum_u = 0;
-    bool found = false;
-    for (int mf = 0; !found;) {
-      R min_m = num<R>::inf(), max_m = -num<R>::inf(), sum_m = 0, num_m_sum_u = 0;
-      R den = k_u * k_u;
-      const R k_u_sum_u = k_u * sum_u;
-      for (int ml = mf;;) {
-        const R tt_ = (num_u * sum_m - k_u_sum_u) / den;
-        const R hh = (num_m_sum_u + k_u * sum_m) / den;
-        const R tt = hh + tt_;
-        if (max_m - eps16 <= tt && tt <= min_u + eps16 && tt_ <= min_m + eps16 &&
-            (ml == mp || static_cast<R>(s[ml]) - eps16 <= tt_)) {
-          t = tt_;
-          th = hh;
-          f = mf;
-          l = ml;
-          found = true;
-          break;
-        }
-        if (ml == mp) break;
-        min_m = static_cast<R>(s[ml]);
-        max_m = static_cast<R>(s[mf]);
-        sum_m += min_m;
-        num_m_sum_u += sum_u;
-        den += num_u;
-        ++ml;
-      }
-      if (found || mf == k) break;
-      min_u = static_cast<R>(s[mf]);
-      sum_u += min_u;
-      k_u -= R(1);
-      num_u += R(1);
-      ++mf;
-    }
-    if (!found) return R(0);  // default zero thresholds
-  }
-  if (!lt) {
-    // The knapsack's root: the threshold formed from the final free range
-    // and the loss summed entry by entry minus t (sum p - gamma), as the
-    // register epilogue does (set_threshold, clamp_loss).
-    if (l > f)
-      t = (sorted_sum<D, R>(s, f, l) + static_cast<R>(f) * hi - gamma) / static_cast<R>(l - f);
+  if (branch == SDCA_BRANCH_KNAPSACK) {
+    // The knapsack's root: the loss summed entry by entry minus
+    // t (sum p - gamma), as the register epilogue does (set_threshold,
+    // clamp_loss).
     double hp = 0, pp = 0, sp = 0;
-    for (int q = 0; q < mp; ++q) {
+    for (int q = lane; q < mp; q += 64) {
       const R x = static_cast<R>(s[q]);
       const R p = clamp_ref(x - t, R(0), hi);
       hp += static_cast<double>(x * p);
       pp += static_cast<double>(p * p);
       sp += static_cast<double>(p);
     }
+    hp = wave_total(hp);
+    pp = wave_total(pp);
+    sp = wave_total(sp);
     return static_cast<R>(hp) - R(0.5) * static_cast<R>(pp) - t * (static_cast<R>(sp) - gamma);
   }
+  const int l = f + n_mid;
+  double dot = 0;
+  for (int q = f + lane; q < l; q += 64) {
+    const double x = static_cast<double>(static_cast<R>(s[q]));
+    dot += x * x;
+  }
   SetStats<R> st;
-  st.sum_u = sorted_sum<D, R>(s, 0, f);
+  st.sum_u = sum_range<R>(s, 0, f);
   st.n_u = f;
-  st.sum_m = sorted_sum<D, R>(s, f, l);
-  st.dot_m = sorted_dot<D, R>(s, f, l);
-  st.n_m = l - f;
-  return smooth_loss(t, th, st);
+  st.sum_m = sum_range<R>(s, f, l);
+  st.dot_m = static_cast<R>(wave_total(dot));
+  st.n_m = n_mid;
+  return smooth_loss(t, hi, st);
 }
 
 template <class D, class R>
@@ -1033,10 +947,10 @@ eval_slow_kernel(const D* __restrict__ S, const int64_t* __restrict__ labels, in
         __syncthreads();
       }
     }
-    if (threadIdx.x == 0) {
+    if (threadIdx.x < 64) {
       const EvalObj ob = objs.o[o];
-      per_example[(i * objs.n + o) * 2] = static_cast<double>(
-          smooth_topk_sorted<D, R>(s, m - 1, ob.k, static_cast<R>(ob.gamma)));
+      const R loss = smooth_topk_sorted<D, R>(s, m - 1, ob.k, static_cast<R>(ob.gamma));
+      if (threadIdx.x == 0) per_example[(i * objs.n + o) * 2] = static_cast<double>(loss);
     }
     __syncthreads();
   }
@@ -1437,10 +1351,30 @@ reduce_final_kernel(const double* __restrict__ partials, int nb, int n_obj,
   }
 }
 
+// hist[c] = #{i: counts[i] == c}: each workgroup counts its share in LDS and
+// adds its bins once (kHistBins; the counts of a trained model fall into a
+// few bins, whose global atomics one by one took 71 us for 20,000 examples,
+// 5 us so).  More bins than that go to memory directly.
+constexpr int kHistBins = 4096;
+
 __global__ void __launch_bounds__(256)
-hist_kernel(const int* __restrict__ counts, int64_t n, unsigned long long* __restrict__ hist) {
-  for (int64_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += static_cast<int64_t>(gridDim.x) * 256)
-    atomicAdd(hist + counts[i], 1ull);
+hist_kernel(const int* __restrict__ counts, int64_t n, int64_t m,
+            unsigned long long* __restrict__ hist) {
+  __shared__ unsigned bins[kHistBins];
+  const bool local = m <= kHistBins;
+  if (local) {
+    for (int b = threadIdx.x; b < m; b += 256) bins[b] = 0;
+    __syncthreads();
+  }
+  for (int64_t i = blockIdx.x * 256ll + threadIdx.x; i < n; i += static_cast<int64_t>(gridDim.x) * 256) {
+    if (local) atomicAdd(bins + counts[i], 1u);
+    else atomicAdd(hist + counts[i], 1ull);
+  }
+  if (local) {
+    __syncthreads();
+    for (int b = threadIdx.x; b < m; b += 256)
+      if (bins[b]) atomicAdd(hist + b, static_cast<unsigned long long>(bins[b]));
+  }
 }
 
 __global__ void zero_u64_kernel(unsigned long long* p, int64_t count) {
@@ -1627,10 +1561,10 @@ hipError_t launch_eval_reduce(const EvalLaunch& a, double* sums, double* rank_su
                        a.stream, hist, a.m);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
-    int64_t blocks = (a.n + 255) / 256;
-    if (blocks > 4096) blocks = 4096;
+    const int64_t blocks = a.m <= kHistBins ? std::min<int64_t>(256, (a.n + 2047) / 2048)
+                                            : std::min<int64_t>(4096, (a.n + 255) / 256);
     hipLaunchKernelGGL(hist_kernel, dim3(static_cast<unsigned>(blocks > 0 ? blocks : 1)), dim3(256),
-                       0, a.stream, a.counts, a.n, hist);
+                       0, a.stream, a.counts, a.n, a.m, hist);
     e = hipGetLastError();
   }
   return e;

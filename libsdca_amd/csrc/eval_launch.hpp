@@ -88,6 +88,13 @@ hipError_t launch_eval_reduce(const EvalLaunch& a, double* sums, double* rank_su
 hipError_t launch_regularizer(int data, const void* W, const void* W0, int64_t count,
                               double* partials, double* out, hipStream_t stream);
 
+// W = W0 + X A' (W0 may be NULL) with ws of primal_workspace_values values:
+// the examples split over the chip, no transposed copies (eval_primal.hip),
+// for the shapes primal_split says.
+bool primal_split(int data, int64_t d, int64_t m, int64_t n);
+int64_t primal_workspace_values(int64_t d, int64_t m, int64_t n);
+hipError_t launch_primal(int data, const void* X, const void* A, const void* W0, void* W, void* ws,
+                         int64_t d, int64_t m, int64_t n, hipStream_t stream);
 // out (cols x rows) = in (rows x cols)^T, both row-major.
 hipError_t launch_transpose(int data, const void* in, void* out, int64_t rows, int64_t cols,
                             hipStream_t stream);

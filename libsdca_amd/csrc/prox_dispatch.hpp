@@ -83,7 +83,7 @@ hipError_t launch_one(const ProxLaunch& a) {
 // threads, kMaxWideThreads for the largest fp32 columns), C slots per
 // thread; the column (at most kMaxColumnBytes) is staged in LDS and the
 // group reductions combine the waves through LDS.  (The knapsack, 40e6 fp32
-// entries: m = 3000 144 us, 8000 88, 16000 105, 30000 160, against 2286,
+// entries: m = 3000 359 us, 8000 249, 16000 324, 30000 417, against 2286,
 // 2495, 4893 and 11745 with the column sorted in LDS.)
 template <int FAM, int KM, class D, class R>
 hipError_t launch_wide(const ProxLaunch& a) {

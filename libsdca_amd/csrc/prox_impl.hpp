@@ -159,8 +159,15 @@ __device__ inline KnapState<R> knapsack_eq_regs(const D (&v)[C], int m, int nval
       w[c] = x;
     }
   };
+  // SEQ: the sums rounded to R once and IEEE quotients, the sorted column's
+  // own roundings (knapsack_sorted), so that both end with the same sets.
+  constexpr bool SEQ = sizeof(S) > sizeof(R);
+  auto quotient = [](R n, R d) -> R {
+    if constexpr (SEQ) return n / d;
+    else return div_near(n, d);
+  };
   int mc = m - n_u0;
-  R t = div_near(total - sum_u0 - rhs + static_cast<R>(n_u0) * hi, static_cast<R>(mc));
+  R t = quotient(total - sum_u0 - rhs + static_cast<R>(n_u0) * hi, static_cast<R>(mc));
   R t_acc = t;
   bool have_acc = false;
   int n_f = 0;
@@ -178,18 +185,19 @@ __device__ inline KnapState<R> knapsack_eq_regs(const D (&v)[C], int m, int nval
   }
   for (int iter = 0; iter <= m; ++iter) {
     const R c_lo = lo + t, c_hi = hi + t;
-    R s_lo = 0, s_hi = 0;
+    S sum_lo = 0, sum_hi = 0;
     int n_lh = 0;
 #pragma unroll UW
     for (int c = 0; c < C; ++c) {
       const R wc = get(c);
       const bool lo_c = wc <= c_lo;
       const bool hi_c = wc > c_hi;
-      s_lo += lo_c ? wc : R(0);
-      s_hi += hi_c ? wc : R(0);
+      sum_lo += lo_c ? wc : R(0);
+      sum_hi += hi_c ? wc : R(0);
       n_lh += (lo_c ? 1 : 0) + (hi_c ? 0x10000 : 0);
     }
-    group_sums<G>(s_lo, s_hi, n_lh);
+    group_sums<G>(sum_lo, sum_hi, n_lh);
+    const R s_lo = static_cast<R>(sum_lo), s_hi = static_cast<R>(sum_hi);
     const int n_lo = n_lh & 0xffff, n_hi = static_cast<int>(static_cast<unsigned>(n_lh) >> 16);
     const R sh = static_cast<R>(n_hi) * hi;
     const R sl = static_cast<R>(n_lo) * lo;
@@ -223,7 +231,7 @@ __device__ inline KnapState<R> knapsack_eq_regs(const D (&v)[C], int m, int nval
       put(c, fixed ? qnan : wc);
     }
     if (mc > 0) {
-      t = div_near(next, static_cast<R>(mc));
+      t = quotient(next, static_cast<R>(mc));
     } else {
       break;
     }
@@ -249,7 +257,11 @@ __device__ inline KnapState<R> knapsack_eq_regs(const D (&v)[C], int m, int nval
     }
     s_f = group_sum<G>(s_f);
     const int n_l = m - st.n_u - n_f;
-    t_acc = static_cast<R>(div_near(s_f + static_cast<S>(st.n_u) * static_cast<S>(hi) +
+    if constexpr (SEQ)
+      t_acc = (static_cast<R>(s_f) + static_cast<R>(st.n_u) * hi + static_cast<R>(n_l) * lo - rhs) /
+              static_cast<R>(n_f);
+    else
+      t_acc = static_cast<R>(div_near(s_f + static_cast<S>(st.n_u) * static_cast<S>(hi) +
                                         static_cast<S>(n_l) * static_cast<S>(lo) -
                                         static_cast<S>(rhs),
                                     static_cast<S>(n_f)));
@@ -351,16 +363,18 @@ __device__ inline ColThr<R> knap_family(const D (&v)[C], int m, int nvalid,
   }
   KnapState<R> st;
   R total = 0;
-  // Columns held by a workgroup of 512 threads or more sum their final free
-  // set in double.
+  // Columns held by a workgroup of 512 threads or more sum in double.
   typedef typename std::conditional<(G >= 512), double, R>::type S;
   // With lo = 0 and hi >= rhs the largest entry alone can take the whole
   // sum, so t >= max - rhs: the entries below that bound end at 0 and are
   // left out (as padding) from the start.  Kiwiel's start at the mean halves
   // the free set about once per pass instead; what remains above the bound
   // of an N(0,1) column is a handful of entries (40e6 fp32 entries: m = 100
-  // 87 -> 63 us, 300 174 -> 128, 1000 103 -> 68).
-  const bool from_max = lo == R(0) && hi >= rhs;
+  // 87 -> 63 us, 300 174 -> 128, 1000 103 -> 68).  Not for a workgroup's
+  // float column: there the rounding of the fixing's numerator (sums of
+  // thousands over a dozen free values) decides which values near t are free,
+  // and it takes the sorted column's steps from the mean on.
+  const bool from_max = lo == R(0) && hi >= rhs && sizeof(S) == sizeof(R);
   if (from_max) {
     R mx = -num<R>::inf();
 #pragma unroll
@@ -381,7 +395,7 @@ __device__ inline ColThr<R> knap_family(const D (&v)[C], int m, int nvalid,
     group_sums<G>(s_c, n_c);
     st = knapsack_eq_regs<G, C, D, R, false, S>(w, n_c, nvalid, s_c, lo, hi, rhs);
   } else {
-    total = total_sum<G, C, D, R>(v, nvalid);
+    total = static_cast<R>(total_sum<G, C, D, S>(v, nvalid));
     st = knapsack_eq_regs<G, C, D, R, false, S>(v, m, nvalid, total, lo, hi, rhs);
   }
   if (biased) {

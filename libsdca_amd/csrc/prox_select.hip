@@ -22,8 +22,8 @@
 // that the fixed work per column (two sorts of 64 values, the searches).
 // Measured on MI355X, 40e6 fp32 entries, us per launch, sorting the whole
 // column -> selection:
-//   top-k simplex k = 10:  m = 700 2568 -> 92, 1000 1875 -> 70,
-//                          1500 2261 -> 64, 8000 2523 -> 74, 30000 11841 -> 79
+//   top-k simplex k = 10:  m = 700 2568 -> 92, 1000 1875 -> 70, 1500 2261 -> 64
+//   top-k simplex k = 5, 4096 columns of 10,000:  7355 -> 343
 //   top-k cone k = 5 on margins (U/M searches):  m = 100 12812 -> 653,
 //                          1000 15076 -> 443, 3000 7918 -> 105
 // (one read and one write of them take 52 us at the rate of a large copy
@@ -33,24 +33,20 @@
 // (prox_sorted.hpp).
 #include <algorithm>
 #include <climits>
+#include <type_traits>
 
 #include "common.hpp"
 #include "prox_impl.hpp"
 #include "prox_launch.hpp"
+#include "prox_select.hpp"
 #include "prox_sorted.hpp"
 
 namespace sdca_gpu {
 
 namespace {
 
-// Most values of the sorted list (four per lane of a wave).
-constexpr int kSelectMax = 256;
 // Waves per workgroup of the wave-per-column form.
 constexpr int kSelectWaves = 4;
-// Part maxima whose rank gives the cut for a search that may need more than
-// the k + 1 largest: about 64 log(64 / (64 - r)) values lie above the r-th.
-constexpr int kSearchRank = 24;
-constexpr int kSearchRankLast = 56;
 
 // Group-wide synchronisation of a column's LDS.
 template <int BT>
@@ -61,283 +57,6 @@ __device__ inline void select_sync() {
 template <int BT>
 __device__ inline int select_lane() {
   return static_cast<int>(threadIdx.x) & (BT > 64 ? BT - 1 : 63);
-}
-
-// Descending bitonic sort of a wave's 64 * CC values, element l * CC + c in
-// slot c of lane l; each compare-exchange is one median with a bound of +inf
-// (keep the larger) or -inf (keep the smaller), as in group_sort_desc.
-template <int SIZE, int STRIDE, int CC, class D>
-__device__ inline void wave_sort_stage(D (&x)[CC], int lane, D pinf) {
-  constexpr int N = 64 * CC;
-  if constexpr (STRIDE < CC) {
-#pragma unroll
-    for (int c = 0; c < CC; ++c) {
-      if ((c & STRIDE) == 0) {
-        const bool desc = SIZE >= N || (SIZE < CC ? (c & SIZE) == 0 : (lane & (SIZE / CC)) == 0);
-        const D a = x[c], b = x[c + STRIDE];
-        const D bound = desc ? pinf : -pinf;
-        x[c] = max_or_min(a, b, bound);
-        x[c + STRIDE] = max_or_min(a, b, -bound);
-      }
-    }
-  } else {
-    constexpr int L = STRIDE / CC;
-    const bool desc = SIZE >= N || (lane & (SIZE / CC)) == 0;
-    const D bound = (desc == ((lane & L) == 0)) ? pinf : -pinf;
-#pragma unroll
-    for (int c = 0; c < CC; ++c) x[c] = max_or_min(x[c], xor_lane<L, true>(x[c]), bound);
-  }
-  if constexpr (STRIDE > 1) wave_sort_stage<SIZE, STRIDE / 2, CC>(x, lane, pinf);
-}
-template <int SIZE, int CC, class D>
-__device__ inline void wave_sort_from(D (&x)[CC], int lane, D pinf) {
-  wave_sort_stage<SIZE, SIZE / 2, CC>(x, lane, pinf);
-  if constexpr (SIZE < 64 * CC) wave_sort_from<2 * SIZE, CC>(x, lane, pinf);
-}
-template <int CC, class D>
-__device__ inline void wave_sort_desc(D (&x)[CC]) {
-  wave_sort_from<2, CC>(x, static_cast<int>(threadIdx.x) & 63, net_inf(D(0)));
-}
-
-// Exclusive prefix sum over the wave (as wave_exclusive_scan_dpp).
-__device__ inline double wave_exclusive_scan(double x) {
-  double incl = x;
-  incl = dpp_add<0x111, 0xF, true>(incl);   // row_shr:1
-  incl = dpp_add<0x112, 0xF, true>(incl);   // row_shr:2
-  incl = dpp_add<0x114, 0xF, true>(incl);   // row_shr:4
-  incl = dpp_add<0x118, 0xF, true>(incl);   // row_shr:8
-  incl = dpp_add<0x142, 0xA, false>(incl);  // row_bcast:15
-  incl = dpp_add<0x143, 0xC, false>(incl);  // row_bcast:31
-  return incl - x;
-}
-
-// The list's cnt <= 64 CC values sorted in place, and ps[i] = the sum of its
-// first i values in double, i <= cnt.  One wave.
-template <int CC, class D>
-__device__ inline void list_sort(D* list, double* ps, int cnt) {
-  const int lane = static_cast<int>(threadIdx.x) & 63;
-  D x[CC];
-#pragma unroll
-  for (int c = 0; c < CC; ++c) {
-    const int i = lane * CC + c;
-    x[c] = (i < cnt) ? list[i] : -num<D>::inf();
-  }
-  wave_sort_desc<CC>(x);
-  double tot = 0;
-#pragma unroll
-  for (int c = 0; c < CC; ++c) tot += (lane * CC + c < cnt) ? static_cast<double>(x[c]) : 0.0;
-  double run = wave_exclusive_scan(tot);
-  wave_lds_sync();
-#pragma unroll
-  for (int c = 0; c < CC; ++c) {
-    const int i = lane * CC + c;
-    if (i < cnt) {
-      list[i] = x[c];
-      ps[i] = run;
-      run += static_cast<double>(x[c]);
-      if (i == cnt - 1) ps[cnt] = run;
-    }
-  }
-  wave_lds_sync();
-}
-
-// The record of a column, or why there is none yet.
-enum { SEL_DONE = 0, SEL_FIX = 1, SEL_U0 = 2, SEL_WIDER = 3, SEL_SLOW = 4 };
-template <class R>
-struct SelectRecord {
-  R t, hi;
-  int state, branch, n_hi, n_mid;
-};
-
-// The partition of the knapsack sum_i clamp(a_i - t, 0, hi) = rhs on the
-// sorted list (every value above t is in it): rank r is above t where
-// f(a_r) < rhs and at hi where f(a_r - hi) <= rhs, one rank per lane, f from
-// the prefix sums and a binary search for the ranks at hi (or inside) at
-// that point.  The same eps as the fixing's (topk_sorted_root).  The
-// threshold is formed from the direct sum over the free ranks; with none
-// free any t of [a_u, a_(u-1) - hi] is the same projection and the record
-// takes the middle.
-template <class D, class R>
-__device__ inline void list_knapsack(const D* list, const double* ps, int cnt, int m, D cut, R hi_r,
-                                     R rhs_r, R& t_out, int& u_out, int& e_out) {
-  const int lane = static_cast<int>(threadIdx.x) & 63;
-  const double hi = static_cast<double>(hi_r), rhs = static_cast<double>(rhs_r);
-  const double eps = static_cast<double>(num<R>::eps() * dmax(R(1), fabs(rhs_r)));
-  int e = 0, u = 0;
-  for (int base = 0; base < cnt; base += 64) {
-    const int r = base + lane;
-    bool above = false, at_hi = false;
-    if (r < cnt) {
-      const double a = static_cast<double>(list[r]);
-      int b = 0, w = r;
-      while (b < w) {  // ranks above a + hi
-        const int mid = (b + w) >> 1;
-        if (static_cast<double>(list[mid]) > a + hi) b = mid + 1;
-        else w = mid;
-      }
-      above = ps[r] - ps[w] - static_cast<double>(r - w) * a + static_cast<double>(w) * hi < rhs - eps;
-      int z = cnt;
-      b = r + 1;
-      while (b < z) {  // ranks above a - hi
-        const int mid = (b + z) >> 1;
-        if (static_cast<double>(list[mid]) > a - hi) b = mid + 1;
-        else z = mid;
-      }
-      at_hi = static_cast<double>(r + 1) * hi + (ps[z] - ps[r + 1]) -
-                  static_cast<double>(z - r - 1) * (a - hi) <= rhs + eps;
-    }
-    e += __popcll(__ballot(above));
-    u += __popcll(__ballot(at_hi));
-    if (base + 64 > e && base + 64 > u) break;  // no later rank is above t
-  }
-  if (u > e) u = e;
-  if (e > u) {
-    double s = 0;
-    for (int i = u + lane; i < e; i += 64) s += static_cast<double>(list[i]);
-    s = wave_total(s);
-    t_out = static_cast<R>((s + static_cast<double>(u) * hi - rhs) / static_cast<double>(e - u));
-  } else {
-    const double top = (u > 0 ? static_cast<double>(list[u - 1]) : static_cast<double>(list[0])) - hi;
-    double low = top;
-    if (u < cnt) low = static_cast<double>(list[u]);
-    else if (u < m) low = static_cast<double>(cut);
-    t_out = static_cast<R>(0.5 * (low + top));
-  }
-  u_out = u;
-  e_out = e;
-}
-
-// topk_cone_search (topk_cone.h:58-133) and its biased form
-// (topk_cone_biased.h:9-106) on the sorted list, from |U| = u_first on: for
-// each |U| = u the candidate ends e of M = ranks [u, e) are tried by the
-// lanes, the smallest accepted e of the smallest u wins, as in the
-// reference's order.  The list holds the column's cnt largest values, the
-// others are at most `cut`.  Where a search for some u may continue past
-// the list (no end accepted, and t not certainly above every M that would;
-// the bound of cone_biased_regs) the result is SEL_WIDER.
-template <class D, class R>
-__device__ inline SelectRecord<R> list_cone(const D* list, const double* ps, int cnt, int m, D cut,
-                                            int k, R rho, int u_first) {
-  const int lane = static_cast<int>(threadIdx.x) & 63;
-  const R eps = R(16) * num<R>::eps();
-  const R K = static_cast<R>(k);
-  SelectRecord<R> rec;
-  rec.state = SEL_DONE;
-  rec.branch = SDCA_BRANCH_SCAN;
-  for (int u = u_first; u <= k; ++u) {
-    const R k_u = static_cast<R>(k - u);
-    const R nu = rho * K * K + static_cast<R>(u);
-    const double pu = ps[u];
-    const R sum_u = static_cast<R>(pu);
-    const R min_u = u > 0 ? static_cast<R>(list[u - 1]) : num<R>::inf();
-    const R first = u < cnt ? static_cast<R>(list[u]) : -num<R>::inf();
-    for (int e0 = u;; e0 += 64) {
-      const int e = e0 + lane;
-      const bool in = e <= cnt;
-      const int ei = in ? e : cnt;
-      const R n_m = static_cast<R>(ei - u);
-      const R sum_m = static_cast<R>(ps[ei] - pu);
-      const R den = k_u * k_u + n_m * nu;
-      const R t = (nu * sum_m - k_u * sum_u) / den;
-      const R hi = (n_m * sum_u + k_u * sum_m) / den;
-      const R max_m = ei > u ? first : -num<R>::inf();
-      const R min_m = ei > u ? static_cast<R>(list[ei - 1]) : num<R>::inf();
-      const R tt = hi + t;
-      const bool pass = in && max_m - eps <= tt && tt <= min_u + eps && t <= min_m + eps;
-      const R next = ei < cnt ? static_cast<R>(list[ei]) : static_cast<R>(cut);
-      const bool take = pass && (ei == m || next - eps <= t);
-      const unsigned long long taken = __ballot(take);
-      if (taken) {
-        const int l = __ffsll(taken) - 1;
-        rec.t = read_lane(t, __builtin_amdgcn_readfirstlane(l));
-        rec.hi = read_lane(hi, __builtin_amdgcn_readfirstlane(l));
-        rec.n_hi = u;
-        rec.n_mid = e0 + l - u;
-        return rec;
-      }
-      // Nothing accepted up to e: where t is certainly above every later
-      // min(M) (the bound above, next the largest value still to come), the
-      // search for this u is over.
-      const R tol = R(2) * eps + R(8) * num<R>::eps() * dmax(fabs(t), fabs(next));
-      const bool ends = den * (t - next) > tol * (den + static_cast<R>(m - ei) * nu);
-      if (e0 + 64 > cnt) {
-        if (cnt < m && __ballot(in && e == cnt && (pass || !ends))) {
-          rec.state = SEL_WIDER;
-          return rec;
-        }
-        break;
-      }
-      if (__ballot(in && ends)) break;
-    }
-  }
-  rec.t = rec.hi = R(0);
-  rec.branch = SDCA_BRANCH_DEFAULT;
-  rec.n_hi = rec.n_mid = 0;
-  return rec;
-}
-
-// The record from the sorted list (list_sort): thresholds_topk_cone,
-// thresholds_topk_simplex and the biased forms (topk_cone.h:18-157,
-// topk_simplex.h:39-68, topk_simplex_biased.h:40-71,
-// topk_cone_biased.h:98-113).  complete: every value above the knapsack's
-// threshold is in the list (otherwise the special cases only, and SEL_FIX).
-template <class D, class R>
-__device__ inline SelectRecord<R> list_record(const D* list, const double* ps, int cnt, int m, D cut,
-                                              const ProxParamsT<R>& pp, bool complete) {
-  const int k = pp.k;
-  const R K = static_cast<R>(k);
-  const R rho = pp.rho, rhs = pp.rhs;
-  const R eps16 = R(16) * num<R>::eps();
-  const bool cone = pp.op == OP_TOPK_CONE || pp.op == OP_TOPK_CONE_BIASED;
-  SelectRecord<R> rec;
-  rec.state = SEL_DONE;
-  rec.t = rec.hi = R(0);
-  rec.branch = SDCA_BRANCH_ZERO;
-  rec.n_hi = rec.n_mid = 0;
-  const R sum_k = static_cast<R>(ps[k]);
-  if (sum_k <= eps16) return rec;
-  const R hi_c = sum_k / (K + rho * K * K);
-  const R t_c = static_cast<R>(list[k - 1]) - hi_c;
-  const bool constant = k == m || t_c >= static_cast<R>(list[k < cnt ? k : k - 1]) - eps16;
-  const R eps = num<R>::eps() * dmax(R(1), fabs(rhs));
-  if (constant && (cone || !(K * hi_c > rhs + eps))) {
-    rec.t = t_c;
-    rec.hi = hi_c;
-    rec.branch = SDCA_BRANCH_CONSTANT;
-    rec.n_hi = k;
-    return rec;
-  }
-  if (!cone) {
-    if (!complete) {
-      rec.state = SEL_FIX;
-      return rec;
-    }
-    int u, e;
-    list_knapsack<D, R>(list, ps, cnt, m, cut, pp.rhs_k, rhs, rec.t, u, e);
-    bool lt = false;
-    if (!constant) {
-      if (u == 0) {
-        lt = rec.t < rho * rhs - eps;
-      } else {
-        const R num_u = static_cast<R>(u);
-        lt = K * (static_cast<R>(ps[u]) + (K - num_u) * rec.t) < rhs * (num_u + rho * K * K) - eps;
-      }
-    }
-    if (!lt) {
-      rec.hi = pp.rhs_k;
-      rec.branch = SDCA_BRANCH_KNAPSACK;
-      rec.n_hi = u;
-      rec.n_mid = e - u;
-      return rec;
-    }
-  }
-  // Without the bias the search's U = 0 partition is every value above 16
-  // eps: its sum needs the whole column.
-  if (rho == R(0)) {
-    rec.state = SEL_U0;
-    return rec;
-  }
-  return list_cone<D, R>(list, ps, cnt, m, cut, k, rho, 0);
 }
 
 template <class D, class R, int BT, int C>
@@ -351,6 +70,12 @@ prox_select_kernel(const D* __restrict__ in, D* __restrict__ out, int64_t m64, i
   __shared__ D sh_cut[BT > 64 ? 1 : kSelectWaves];
   __shared__ int sh_cnt[2];  // the workgroup's compaction counter, two in turn
   constexpr int NG = BT > 64 ? 1 : kSelectWaves;  // groups per workgroup
+  // A float workgroup's column (of more than 2048 values) whose sets rounding
+  // decides takes the sorted column's steps: with the numerator at sums of
+  // thousands, a dozen values free, they place t a hundred ulps off, and a
+  // result should not depend on the path its column takes.
+  constexpr bool kClose = BT > 64 && sizeof(R) == 4;
+  __shared__ R sh_mag[kClose ? BT / 64 : 1];
   const int grp = BT > 64 ? 0 : static_cast<int>(threadIdx.x) >> 6;
   const int lane = static_cast<int>(threadIdx.x) & 63;
   const bool lead = BT == 64 || threadIdx.x < 64;  // the wave that solves
@@ -376,6 +101,7 @@ prox_select_kernel(const D* __restrict__ in, D* __restrict__ out, int64_t m64, i
     asm("" : "+v"(tid));
     D v[C];
     bool finite = true;
+    R mag = 0;  // sum |a_i|, for the test of a close call (kClose)
     if (vec) {
       constexpr int E = 16 / static_cast<int>(sizeof(D));
       typedef D word __attribute__((ext_vector_type(E)));
@@ -387,6 +113,7 @@ prox_select_kernel(const D* __restrict__ in, D* __restrict__ out, int64_t m64, i
 #pragma unroll
         for (int l = 0; l < E; ++l) {
           finite = finite && fabs(x[l]) < num<D>::inf();
+          if constexpr (kClose) mag += ok ? static_cast<R>(fabs(x[l])) : R(0);
           v[q * E + l] = ok ? x[l] : -num<D>::inf();
         }
       }
@@ -396,6 +123,7 @@ prox_select_kernel(const D* __restrict__ in, D* __restrict__ out, int64_t m64, i
         const int i = c * BT + tid;
         const D x = col[i < m ? i : 0];
         finite = finite && fabs(x) < num<D>::inf();
+        if constexpr (kClose) mag += i < m ? static_cast<R>(fabs(x)) : R(0);
         v[c] = i < m ? x : -num<D>::inf();
       }
     }
@@ -407,6 +135,10 @@ prox_select_kernel(const D* __restrict__ in, D* __restrict__ out, int64_t m64, i
     if (!finite) part = num<D>::inf();  // seen below: the column goes to the sort
     if constexpr (BT > 64) {
       parts[threadIdx.x] = part;
+      if constexpr (kClose) {
+        mag = wave_total(mag);
+        if (lane == 0) sh_mag[threadIdx.x >> 6] = mag;
+      }
       if (threadIdx.x == 0) sh_cnt[0] = sh_cnt[1] = 0;
       __syncthreads();
       if (lead) {
@@ -414,6 +146,11 @@ prox_select_kernel(const D* __restrict__ in, D* __restrict__ out, int64_t m64, i
         for (int i = 1; i < BT / 64; ++i) {
           const D y = parts[64 * i + lane];
           part = (y > part) ? y : part;
+        }
+        if constexpr (kClose) {
+          mag = R(0);
+#pragma unroll
+          for (int i = 0; i < BT / 64; ++i) mag += sh_mag[i];
         }
       }
     }
@@ -514,6 +251,21 @@ prox_select_kernel(const D* __restrict__ in, D* __restrict__ out, int64_t m64, i
         else if (cnt <= 128) list_sort<2>(list, ps, cnt);
         else list_sort<4>(list, ps, cnt);
         rec = list_record<D, R>(list, ps, cnt, m, cut, pp, cone || attempt != 1);
+        if constexpr (kClose) {
+          // The fixing's numerator sums up to sum |a_i| in R, so its
+          // threshold strays by a few ulps of that over the free values; a
+          // value so near to t or t + hi may fall on either side there.
+          if (rec.state == SEL_DONE && rec.branch == SDCA_BRANCH_KNAPSACK) {
+            const R stray = num<R>::eps() * mag / static_cast<R>(rec.n_mid);
+            const int u = rec.n_hi, e = rec.n_hi + rec.n_mid;
+            const R low = static_cast<R>(e < cnt ? list[e] : cut);
+            // (none free: the fixing keeps its t)
+            if (e == u || (u > 0 && static_cast<R>(list[u - 1]) - rec.t - rec.hi < stray) ||
+                rec.t + rec.hi - static_cast<R>(list[u]) < stray ||
+                static_cast<R>(list[e - 1]) - rec.t < stray || rec.t - low < stray)
+              rec.state = SEL_FIX;
+          }
+        }
       }
       if constexpr (BT > 64) {
         if (threadIdx.x == 0) rec_lds = rec;
@@ -561,14 +313,24 @@ prox_select_kernel(const D* __restrict__ in, D* __restrict__ out, int64_t m64, i
         }
       }
       if (rec.state == SEL_FIX) {
-        // More candidates than the list holds: variable fixing over the
-        // slots, the free set as the value interval (lc, hc].
+        // Variable fixing over the slots, the free set as the value interval
+        // (lc, hc]: more candidates than the list holds, or a workgroup's
+        // column too close to call (below).  A wave's column starts from the
+        // bound of the k-th value; a workgroup's takes the sorted column's
+        // steps (knapsack_sorted: the same start, the numerator carried on
+        // in R, the sums rounded to R once), so that it ends with the same
+        // sets.
+        typedef typename std::conditional<(BT > 64), double, R>::type S;
         const R hi = pp.rhs_k, rhs = pp.rhs;
         const R eps = num<R>::eps() * dmax(R(1), fabs(rhs));
-        const R kth = static_cast<R>(list[k - 1]);
-        const R slack = (fabs(kth) + hi) * (R(16) * num<R>::eps());
-        R lc = kth - hi - slack, hc = kth + hi + slack;
-        R s_f = 0, s_u = 0;
+        R lc = -num<R>::inf(), hc = num<R>::inf();
+        if constexpr (BT == 64) {
+          const R kth = static_cast<R>(list[k - 1]);
+          const R slack = (fabs(kth) + hi) * (R(16) * num<R>::eps());
+          lc = kth - hi - slack;
+          hc = kth + hi + slack;
+        }
+        S s_f = 0, s_u = 0;
         int n_f = 0, n_u = 0;
 #pragma unroll 4
         for (int i = tid; i < m; i += BT) {
@@ -580,10 +342,12 @@ prox_select_kernel(const D* __restrict__ in, D* __restrict__ out, int64_t m64, i
           n_u += x > hc ? 1 : 0;
         }
         group_sums<BT>(s_f, s_u, n_f, n_u);
-        R t = div_near(s_f + static_cast<R>(n_u) * hi - rhs, static_cast<R>(n_f));
+        R t, t_fix;
+        if constexpr (BT > 64) t = (static_cast<R>(s_f) - rhs) / static_cast<R>(n_f);
+        else t = div_near(s_f + static_cast<R>(n_u) * hi - rhs, static_cast<R>(n_f));
         for (int iter = 0; iter <= m; ++iter) {
           const R c_hi = hi + t;
-          R s_lo = 0, s_hi = 0;
+          S s_lo = 0, s_hi = 0;
           int n_lo = 0, n_hi = 0;
 #pragma unroll 4
           for (int i = tid; i < m; i += BT) {
@@ -595,9 +359,13 @@ prox_select_kernel(const D* __restrict__ in, D* __restrict__ out, int64_t m64, i
             n_hi += (f && x > c_hi) ? 1 : 0;
           }
           group_sums<BT>(s_lo, s_hi, n_lo, n_hi);
-          const R infeas = s_hi + s_lo - static_cast<R>(n_hi) * hi - static_cast<R>(n_hi + n_lo) * t;
+          const R r_lo = static_cast<R>(s_lo), r_hi = static_cast<R>(s_hi);
+          const R sh = static_cast<R>(n_hi) * hi;
+          const R infeas = r_hi + r_lo - sh - static_cast<R>(n_hi + n_lo) * t;
           const bool fix_hi = n_hi > 0 && infeas > eps;
           const bool fix_lo = !fix_hi && n_lo > 0 && infeas < -eps;
+          const R mc = static_cast<R>(n_f);
+          t_fix = t;
           if (fix_hi || (!fix_lo && n_hi > 0)) {
             hc = c_hi;
             n_u += n_hi;
@@ -609,6 +377,11 @@ prox_select_kernel(const D* __restrict__ in, D* __restrict__ out, int64_t m64, i
             n_f -= n_lo;
           }
           if (n_f <= 0) break;
+          if constexpr (BT > 64) {
+            if (fix_hi) t = (mc * t - r_hi + sh) / static_cast<R>(n_f);
+            else if (fix_lo) t = (mc * t - r_lo) / static_cast<R>(n_f);
+          }
+          if (BT > 64 && (fix_hi || fix_lo)) continue;
           s_f = 0;
 #pragma unroll 4
           for (int i = tid; i < m; i += BT) {
@@ -616,13 +389,17 @@ prox_select_kernel(const D* __restrict__ in, D* __restrict__ out, int64_t m64, i
             s_f += (x > lc && x <= hc) ? x : R(0);
           }
           s_f = group_sum<BT>(s_f);
-          t = div_near(s_f + static_cast<R>(n_u) * hi - rhs, static_cast<R>(n_f));
+          if constexpr (BT > 64)
+            t = (static_cast<R>(s_f) + static_cast<R>(n_u) * hi - rhs) / static_cast<R>(n_f);
+          else
+            t = t_fix = div_near(s_f + static_cast<R>(n_u) * hi - rhs, static_cast<R>(n_f));
           if (!fix_hi && !fix_lo) break;
         }
         bool lt;
         const R K = static_cast<R>(k), num_u = static_cast<R>(n_u);
-        if (n_u == 0) lt = t < pp.rho * rhs - eps;
-        else lt = K * (s_u + (K - num_u) * t) < rhs * (num_u + pp.rho * K * K) - eps;
+        if (n_u == 0) lt = t_fix < pp.rho * rhs - eps;
+        else
+          lt = K * (static_cast<R>(s_u) + (K - num_u) * t_fix) < rhs * (num_u + pp.rho * K * K) - eps;
         const R sum_k = static_cast<R>(ps[k]);
         const bool constant = static_cast<R>(list[k - 1]) - sum_k / (K + pp.rho * K * K) >=
                               static_cast<R>(list[k]) - R(16) * num<R>::eps();

@@ -23,7 +23,7 @@
 // Measured on MI355X, 40e6 fp32 entries, us per launch, sorting the whole
 // column -> selection:
 //   top-k simplex k = 10:  m = 700 2568 -> 92, 1000 1875 -> 70, 1500 2261 -> 64
-//   top-k simplex k = 5, 4096 columns of 10,000:  7355 -> 343
+//   top-k simplex k = 5, 4096 columns of 10,000:  7364 -> 296
 //   top-k cone k = 5 on margins (U/M searches):  m = 100 12812 -> 653,
 //                          1000 15076 -> 443, 3000 7918 -> 105
 // (one read and one write of them take 52 us at the rate of a large copy
@@ -59,8 +59,13 @@ __device__ inline int select_lane() {
   return static_cast<int>(threadIdx.x) & (BT > 64 ? BT - 1 : 63);
 }
 
+// (One wave per column, up to 16 slots, fp32: four waves per SIMD, one
+// register fewer than the compiler takes by itself; at three waves k = 10,
+// m = 1000 took 105 us per 50,000 columns instead of 94.  In fp64 the bound
+// spills: m = 1000 124 -> 188 us.)
 template <class D, class R, int BT, int C>
-__global__ void __launch_bounds__(BT > 64 ? BT : 64 * kSelectWaves)
+__global__ void __launch_bounds__(BT > 64 ? BT : 64 * kSelectWaves,
+                                  (BT == 64 && C <= 16 && sizeof(D) + sizeof(R) == 8) ? 4 : 1)
 prox_select_kernel(const D* __restrict__ in, D* __restrict__ out, int64_t m64, int64_t n,
                    ProxParamsT<R> pp, sdca_thresholds* __restrict__ thr, int* __restrict__ slow,
                    int all_columns, int pow2, int group_bytes, int vec,

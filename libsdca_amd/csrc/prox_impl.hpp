@@ -376,20 +376,28 @@ __device__ inline ColThr<R> knap_family(const D (&v)[C], int m, int nvalid,
   // and it takes the sorted column's steps from the mean on.
   const bool from_max = lo == R(0) && hi >= rhs && sizeof(S) == sizeof(R);
   if (from_max) {
-    R mx = -num<R>::inf();
+    R mx = -num<R>::inf(), sum = 0;
 #pragma unroll
-    for (int c = 0; c < C; ++c) mx = (static_cast<R>(v[c]) > mx) ? static_cast<R>(v[c]) : mx;
+    for (int c = 0; c < C; ++c) {
+      const R x = static_cast<R>(v[c]);
+      mx = (x > mx) ? x : mx;
+      sum += c < nvalid ? x : R(0);
+    }
+    // A column that holds an infinity or a NaN (or whose sum overflows)
+    // keeps every entry: the bound says nothing about it.
+    mx = fabs(sum) < num<R>::inf() ? mx : num<R>::inf();
     mx = group_max<G>(mx);
     const R cut = mx - rhs - (fabs(mx) + rhs) * (R(16) * num<R>::eps());
+    const bool every = !(mx < num<R>::inf());
     D w[C];
     R s_c = 0;
     int n_c = 0;
 #pragma unroll
     for (int c = 0; c < C; ++c) {
       const R x = static_cast<R>(v[c]);
-      const bool in = c < nvalid && x >= cut;
+      const bool in = c < nvalid && (every || x >= cut);
       w[c] = in ? v[c] : -num<D>::inf();
-      s_c += in ? x : R(0);
+      s_c += (in && x > -num<R>::inf()) ? x : R(0);
       n_c += in ? 1 : 0;
     }
     group_sums<G>(s_c, n_c);

@@ -26,3 +26,26 @@ def test_knapsack_start_at_the_maximum(cuda, oracle, op, kw, m, dtype, result):
                     ("edge", inputs.edge_columns(m, dtype, 903 + m))]:
         got, thr = run_gpu(op, x, result, cuda, **kw)
         parity(oracle, op, x, got, result, f"{op} {name} m={m}", nthreads=8, thr=thr, **kw)
+
+
+@pytest.mark.parametrize("op", ["knapsack_eq", "knapsack_le"])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("m", [10, 40, 100, 700, 1500])
+def test_values_not_finite(cuda, op, dtype, m):
+    """The bound says nothing about a column with an infinity, a NaN or an
+    overflowing sum: such a column ends as it does from the mean, the start
+    of every other lower bound (-1e-30, below the rounding of any t)."""
+    import torch
+    import libsdca_amd as sd
+    rng = np.random.default_rng(m)
+    x = rng.standard_normal((9, m)).astype(dtype)
+    x[1, 3], x[2, 5], x[3, 7] = np.inf, -np.inf, np.nan
+    x[4], x[5], x[6] = -np.inf, np.nan, np.finfo(dtype).max
+    x[7, 1], x[7, 2] = np.inf, -np.inf
+    a = torch.from_numpy(x).to(cuda)
+    got = sd.prox(op, a.clone()).cpu().numpy()
+    want = sd.prox(op, a.clone(), lo=-1e-30).cpu().numpy()
+    assert (np.isnan(got) == np.isnan(want)).all()
+    # 16 m u: the two starts' sums over a column of m values of unit size
+    tol = 16 * m * float(np.finfo(dtype).eps)
+    assert np.allclose(np.nan_to_num(got), np.nan_to_num(want), rtol=0, atol=tol)

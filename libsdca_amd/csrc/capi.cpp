@@ -107,6 +107,21 @@ int workspace(hipStream_t stream, int slot, size_t bytes, void** out, Workspace*
   return SDCA_OK;
 }
 
+// Whether the deferred-column list (slot 0) of `bytes` can be had: not under
+// graph capture beyond what the stream already has.
+bool list_available(hipStream_t stream, size_t bytes) {
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &cs) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;
+  }
+  if (cs == hipStreamCaptureStatusNone) return true;
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return true;
+  std::lock_guard<std::mutex> lock(g_ws_mutex);
+  return g_ws[std::make_tuple(dev, stream, std::this_thread::get_id())].cap[0] >= bytes;
+}
+
 // The library GEMM's workspace (slot 5) for an fp32 score GEMM of n m d:
 // none below the library's threshold, and under graph capture only one the
 // stream already has (the GEMM then takes an algorithm within it, or the
@@ -429,9 +444,14 @@ int prox_entry(int op_in, int data_in, int result_in, int64_t m, int64_t n, cons
     SDCA_HIP_TRY(launch_two_ent(a), "two_entropy kernel (wave per column)");
   } else if (ent_biased) {
     SDCA_HIP_TRY(launch_ent_biased(a), "topk_entropy_biased kernel (wave per column)");
-  } else if (topk_like && !topk_in_registers(op, data, m, p.k)) {
+  } else if (topk_like &&
+             (!topk_in_registers(op, data, m, p.k) ||
+              (p.k > 8 && !fixed_list &&
+               !list_available(stream, static_cast<size_t>(n + 2) * sizeof(int))))) {
     // Columns beyond the register kernel: by selection, or for the largest
-    // k one workgroup per sorted column.
+    // k one workgroup per sorted column.  With k > 8 also where the
+    // register kernel's list of deferred columns would have to be allocated
+    // under capture: these calls need no scratch.
     if (select_supported(a))
       SDCA_HIP_TRY(launch_select(a, true), "prox kernel (selection)");
     else
@@ -443,13 +463,14 @@ int prox_entry(int op_in, int data_in, int result_in, int64_t m, int64_t n, cons
     // reach that kernel.
     Workspace* wsr = nullptr;
     Workspace fixed_ws;  // the fixed scratch's stand-in record (its state is not kept)
-    if (listed && fixed_list) {
+    // (The biased knapsack defers nothing.)
+    if (listed && fixed_list && op != SDCA_PROX_KNAPSACK_LE_BIASED) {
       // The fixed scratch is shared by every call on the device: its two
       // counters are cleared by a kernel on this stream before each use.
       a.slow = fixed_list;
       wsr = &fixed_ws;
       SDCA_HIP_TRY(launch_clear(a.slow, 2, stream), "clear kernel");
-    } else if (listed) {
+    } else if (listed && op != SDCA_PROX_KNAPSACK_LE_BIASED) {
       void* ws = nullptr;
       rc = workspace(stream, 0, static_cast<size_t>(n + 2) * sizeof(int), &ws, &wsr);
       if (rc) return rc;
@@ -477,9 +498,8 @@ int prox_entry(int op_in, int data_in, int result_in, int64_t m, int64_t n, cons
     if (op == SDCA_PROX_TWO_SIMPLEX_SORT) {
       SDCA_HIP_TRY(launch_two_sort(a, false), "two_simplex_sort kernel (deferred columns)");
       wsr->list_zeroed = true;
-    } else if (listed) {
-      // (the biased knapsack defers nothing: its list stays empty)
-      if (topk_like) SDCA_HIP_TRY(launch_select(a, false), "prox kernel (deferred columns)");
+    } else if (topk_like) {
+      SDCA_HIP_TRY(launch_select(a, false), "prox kernel (deferred columns)");
       wsr->list_zeroed = true;
     }
   }

@@ -31,7 +31,6 @@
 #include "prox_impl.hpp"
 #include "prox_lambert_wave.hpp"
 #include "prox_launch.hpp"
-#include "prox_select.hpp"
 #include "prox_sorted.hpp"
 
 namespace sdca_gpu {
@@ -69,11 +68,11 @@ __host__ __device__ constexpr bool epoch_delta_in_lds(int PF) {
   return PF > 0 && (sizeof(D) == 4 ? PF <= 4 : PF <= 1);
 }
 
-// Words of the block's delta rows in LDS: kEpochBlock rows of m (rounded up
-// to 16 bytes where a thread's columns lie side by side) and the padding that the last row's unclamped slot reads run into (the thread
+// Words of the block's delta rows in LDS: kEpochBlock rows of m and the
+// padding that the last row's unclamped slot reads run into (the thread
 // slots cover kEpochThreads PF >= m columns).
 __host__ __device__ inline int epoch_dx_words(int m, int PF) {
-  return kEpochBlock * ((m + 3) & ~3) + (kEpochThreads * PF > m ? kEpochThreads * PF - m : 0);
+  return kEpochBlock * m + (kEpochThreads * PF > m ? kEpochThreads * PF - m : 0);
 }
 
 // Words of the thresholds' column in LDS: m values, or G C for the register
@@ -142,304 +141,18 @@ kernel_at_kernel(const D* __restrict__ A, D* __restrict__ At, const int64_t* __r
 // ok = j < m: the loops stay branch-free (exec-masked branches around each
 // slot cost more than the slot's work), so loads read the clamped column
 // j < m ? j : m - 1 and the stores of slots past m go to the thread's dummy
-// word.  SIDE: the thread's columns lie side by side instead, j = PF tid + q
-// (a delta row is then one 16-byte LDS read per thread).  PF = 0: every
-// j = tid (mod G) below m, q = 0, ok = true.
-template <int PF, bool SIDE = false, class F>
+// word.  PF = 0: every j = tid (mod G) below m, q = 0, ok = true.
+template <int PF, class F>
 __device__ __forceinline__ void for_cols(int tid, int m, F&& f) {
   if constexpr (PF > 0) {
 #pragma unroll
     for (int q = 0; q < PF; ++q) {
-      const int j = SIDE ? PF * tid + q : tid + kEpochThreads * q;
+      const int j = tid + kEpochThreads * q;
       f(j, q, j < m);
     }
   } else {
     for (int j = tid; j < m; j += kEpochThreads) f(j, 0, true);
   }
-}
-
-// The waves' parts of an exchange of two sums and a count.
-template <class R>
-struct EpochSums {
-  R a, b;
-  int n;
-};
-
-// The hinge duals' thresholds (prox_topk_simplex_biased,
-// prox_knapsack_le_biased) of the column spread over the workgroup, w[q] of
-// each thread (-inf where it holds none), by selection as in
-// prox_select.hip: a cut below every value that matters from the maxima of
-// the column's 64 parts (part l: lane l of every wave; parts[] holds the
-// threads' maxima before `shift` was added to the column), the values above
-// it compacted into each wave's share of cand, and the short list solved by
-// all four waves alike, each on its own SIMD: nothing is broadcast.
-//
-// The cut is the knapsack's bound over the part maxima (parts_lower); the
-// list is sorted and solved in the waves' registers (regs_record), through
-// LDS where a search is needed (list_record; the cone search by the sorted
-// column's own chain of sums, whose rounding over M of hundreds of values
-// is part of the result); a knapsack with more
-// candidates than the list holds is solved by variable fixing over the
-// slots; for what is left (state not SEL_DONE) the caller sorts the whole
-// column.
-//
-// What bounds it: the latency of one workgroup's dependent steps.  Measured
-// against each thread keeping a sorted list of its k + 1 largest, merged
-// over the workgroup, and the whole column sorted for every search and k > 8
-// (us per example, all of the epoch's kernels, first epoch | later ones):
-//   m = 1000, d = 4096, k = 5, top-k simplex, fp32   50 -> 30 | 9.1 -> 8.6
-//   m = 1000, d = 512, k = 5, knapsack, fp32          7.4 -> 5.6 | 7.2 -> 5.3
-//   m = 1000, d = 512, k = 10, top-k simplex, fp32    65 -> 18 | 46 -> 5.9
-//   m = 100, d = 512, k = 3, top-k simplex, fp32     15.7 -> 7.8 | 6.7 -> 4.1
-//   m = 800, d = 512, k = 5, top-k simplex, fp64      43 -> 17 | 18 -> 9.5
-template <int PF, class D, class R>
-__device__ __forceinline__ SelectRecord<R> epoch_select(const D (&w)[PF], int mp, D shift,
-                                                        const ProxParamsT<R>& pp, const D* parts,
-                                                        D* cand, D* list, double* ps, int* counts,
-                                                        EpochSums<R>* xs) {
-  constexpr int G = kEpochThreads, NW = G / 64;
-  const int lane = static_cast<int>(threadIdx.x) & 63;
-  const int wave = static_cast<int>(threadIdx.x) >> 6;
-  const bool simplex = pp.op == OP_TOPK_SIMPLEX_BIASED;
-  const R hi = simplex ? pp.rhs_k : pp.hi, rhs = pp.rhs;
-  const R eps = num<R>::eps() * dmax(R(1), fabs(rhs));
-  const int k = pp.k;
-  const bool all = mp <= kSelectMax;  // the column is its own list
-  // The values at or above a cut into cand; returns their number.
-  int first[NW + 1];  // the list position of each wave's first value
-  auto compact = [&](D cut) -> int {
-    int mine = 0;
-#pragma unroll
-    for (int q = 0; q < PF; ++q) {
-      const bool pr = w[q] >= cut;
-      const unsigned long long mask = __ballot(pr);
-      const int at = mine + static_cast<int>(__builtin_amdgcn_mbcnt_hi(
-          static_cast<unsigned>(mask >> 32),
-          __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(mask), 0)));
-      if (pr) cand[wave * 64 * PF + at] = w[q];
-      mine += __popcll(mask);
-    }
-    if (lane == 0) counts[wave] = mine;
-    __syncthreads();
-    first[0] = 0;
-#pragma unroll
-    for (int i = 0; i < NW; ++i)
-      first[i + 1] = first[i] + __builtin_amdgcn_readfirstlane(counts[i]);
-    return first[NW];
-  };
-  // Value i of the list (any order), -inf past its cnt values.
-  auto value = [&](int i, int cnt) -> D {
-    int r = 0, f = 0;
-#pragma unroll
-    for (int j = 1; j < NW; ++j) {
-      r += i >= first[j] ? 1 : 0;
-      f = i >= first[j] ? first[j] : f;
-    }
-    const D x = cand[i < cnt ? r * 64 * PF + i - f : 0];
-    return i < cnt ? x : -num<D>::inf();
-  };
-  D part[1] = {D(0)};
-  if (!all) {
-    D x = parts[lane];
-#pragma unroll
-    for (int i = 1; i < NW; ++i) {
-      const D y = parts[64 * i + lane];
-      x = (y > x) ? y : x;
-    }
-    part[0] = x + shift;
-  }
-  SelectRecord<R> rec;
-  rec.state = SEL_SLOW;
-  rec.t = rec.hi = R(0);
-  rec.branch = rec.n_hi = rec.n_mid = 0;
-  D usual = -num<D>::max_finite(), kth_part = usual;
-  if (!all) {
-    wave_sort_desc<1>(part);
-    kth_part = read_lane(part[0], k);
-    const D lower = parts_lower<D, R>(part, k, hi, rhs);
-    usual = lower < kth_part ? lower : kth_part;
-  }
-  // Sums over the workgroup by one barrier, two buffers in turn.
-  int px = 0;
-  auto exchange = [&](R& a, R& b, int& n) {
-    a = wave_total(a);
-    b = wave_total(b);
-    n = wave_total(n);
-    EpochSums<R>* const x = xs + px * NW;
-    px ^= 1;
-    if (lane == 0) x[wave] = EpochSums<R>{a, b, n};
-    __syncthreads();
-    a = x[0].a;
-    b = x[0].b;
-    n = x[0].n;
-#pragma unroll
-    for (int i = 1; i < NW; ++i) {
-      a += x[i].a;
-      b += x[i].b;
-      n += x[i].n;
-    }
-  };
-  // The usual list (0), or, where that is too long, the special cases' k + 1
-  // largest (1).
-  for (int form = 0; form < 2; ++form) {
-    const D cut = form == 0 ? usual : kth_part;
-    const int cnt = compact(cut);
-    const bool fits = cnt <= kSelectMax && cnt >= (simplex ? min(k + 1, mp) : 1);
-    if (fits) {
-      bool done = false;
-      auto solve = [&](auto& x) {
-        constexpr int CC = sizeof(x) / sizeof(D);
-#pragma unroll
-        for (int c = 0; c < CC; ++c) x[c] = value(lane * CC + c, cnt);
-        wave_sort_desc<CC>(x);
-        if constexpr (CC <= 2) {
-          R rx[CC];
-          regs_prefix<CC, D, R>(x, rx, cnt);
-          if (simplex) {
-            if (form != 1) done = regs_record<CC, D, R>(x, rx, cnt, mp, pp, rec);
-          } else {
-            // knapsack_le_biased.h:102-130: the equality's threshold where it
-            // is at least rho rhs, else the sum constraint is inactive.
-            R sum_u;
-            done = regs_knapsack<CC, D, R>(x, rx, cnt, k, hi, rhs, R(0), rec.t, rec.n_hi, rec.n_mid,
-                                           sum_u);
-            if (done && !(rec.t >= pp.rho * rhs - eps))
-              done = regs_knapsack<CC, D, R>(x, rx, cnt, k, hi, rhs, R(1) / pp.rho, rec.t, rec.n_hi,
-                                             rec.n_mid, sum_u);
-            rec.hi = hi;
-            if (done) rec.state = SEL_DONE;
-          }
-        }
-        if (!done) {
-          double ex[CC];
-          list_prefix<CC>(x, ex, cnt);
-          list_store<CC>(x, ex, list, ps, cnt);
-        }
-      };
-      if (cnt <= 64) {
-        D x[1];
-        solve(x);
-      } else if (cnt <= 128) {
-        D x[2];
-        solve(x);
-      } else {
-        D x[4];
-        solve(x);
-      }
-      if (done) return rec;
-      if (simplex) {
-        rec = list_record<D, R, true>(list, ps, cnt, mp, cut, pp, form != 1);
-      } else {
-        list_knapsack<D, R>(list, ps, cnt, mp, cut, hi, rhs, rec.t, rec.n_hi, rec.n_mid);
-        if (!(rec.t >= pp.rho * rhs - eps))
-          list_knapsack<D, R>(list, ps, cnt, mp, cut, hi, rhs, rec.t, rec.n_hi, rec.n_mid,
-                              R(1) / pp.rho);
-        rec.hi = hi;
-        rec.state = SEL_DONE;
-      }
-      if (rec.state == SEL_DONE) return rec;
-    }
-    // (uniform over the workgroup: every wave holds the same list)
-    if ((fits && rec.state == SEL_FIX) || (!fits && !simplex && cnt > kSelectMax)) {
-      // Variable fixing over the slots, the free set as the value interval
-      // (lc, hc], from the bound of the part maxima; with inv_rho > 0 for
-      // the right side t inv_rho (knapsack_biased_regs).
-      R lc0 = static_cast<R>(usual), hc0 = num<R>::inf();
-      if (simplex) {
-        const R kth = static_cast<R>(list[k - 1]);
-        const R slack = (fabs(kth) + hi) * (R(16) * num<R>::eps());
-        lc0 = dmax(lc0, kth - hi - slack);
-        hc0 = kth + hi + slack;
-      }
-      R t = 0, s_u = 0;
-      int n_f = 0, n_u = 0;
-      auto fixing = [&](R inv_rho) {
-        const R goal = inv_rho > 0 ? R(0) : rhs;
-        R lc = lc0, hc = hc0, s_f = 0;
-        int n_fu = 0;
-        s_u = 0;
-#pragma unroll
-        for (int q = 0; q < PF; ++q) {
-          const R x = static_cast<R>(w[q]);
-          const bool up = x > hc, f = x > lc && !up;
-          s_f += f ? x : R(0);
-          s_u += up ? x : R(0);
-          n_fu += (f ? 1 : 0) + (up ? 0x10000 : 0);
-        }
-        exchange(s_f, s_u, n_fu);
-        n_f = n_fu & 0xffff;
-        n_u = n_fu >> 16;
-        for (int iter = 0; iter <= mp && n_f > 0; ++iter) {
-          t = div_near(s_f + static_cast<R>(n_u) * hi - goal, inv_rho + static_cast<R>(n_f));
-          const R c_hi = hi + t;
-          R s_lo = 0, s_hi = 0;
-          int n_lh = 0;
-#pragma unroll
-          for (int q = 0; q < PF; ++q) {
-            const R x = static_cast<R>(w[q]);
-            const bool f = x > lc && x <= hc;
-            const bool l = f && x <= t, h = f && x > c_hi;
-            s_lo += l ? x : R(0);
-            s_hi += h ? x : R(0);
-            n_lh += (l ? 1 : 0) + (h ? 0x10000 : 0);
-          }
-          exchange(s_lo, s_hi, n_lh);
-          const int n_lo = n_lh & 0xffff, n_hi = n_lh >> 16;
-          const R infeas = s_hi + s_lo - static_cast<R>(n_hi) * hi - static_cast<R>(n_hi + n_lo) * t;
-          const bool fix_hi = n_hi > 0 && infeas > eps;
-          const bool fix_lo = !fix_hi && n_lo > 0 && infeas < -eps;
-          if (!fix_lo && n_hi > 0) {
-            hc = c_hi;
-            n_u += n_hi;
-            s_u += s_hi;
-            n_f -= n_hi;
-            s_f -= s_hi;
-          }
-          if (!fix_hi && n_lo > 0) {
-            lc = t;
-            n_f -= n_lo;
-            s_f -= s_lo;
-          }
-          if (!fix_hi && !fix_lo) break;
-        }
-        if (n_f <= 0) return;
-        // the threshold from the final free set
-        R none = 0;
-        int zero = 0;
-        s_f = 0;
-#pragma unroll
-        for (int q = 0; q < PF; ++q) {
-          const R x = static_cast<R>(w[q]);
-          s_f += (x > lc && x <= hc) ? x : R(0);
-        }
-        exchange(s_f, none, zero);
-        t = div_near(s_f + static_cast<R>(n_u) * hi - goal, inv_rho + static_cast<R>(n_f));
-      };
-      fixing(R(0));
-      if (!simplex && n_f > 0 && !(t >= pp.rho * rhs - eps)) fixing(R(1) / pp.rho);
-      rec.state = n_f > 0 ? SEL_DONE : SEL_SLOW;
-      rec.t = t;
-      rec.hi = hi;
-      if (simplex) {
-        const R K = static_cast<R>(k), num_u = static_cast<R>(n_u);
-        bool lt;
-        if (n_u == 0) lt = t < pp.rho * rhs - eps;
-        else lt = K * (s_u + (K - num_u) * t) < rhs * (num_u + pp.rho * K * K) - eps;
-        const R sum_k = static_cast<R>(ps[k]);
-        const bool constant = static_cast<R>(list[k - 1]) - sum_k / (K + pp.rho * K * K) >=
-                              static_cast<R>(list[k]) - R(16) * num<R>::eps();
-        if (lt && !constant) rec.state = SEL_SLOW;  // the cone search
-      }
-      return rec;
-    }
-    if (fits || form == 1 || !simplex || cnt <= kSelectMax) {
-      rec.state = SEL_SLOW;
-      return rec;
-    }
-    __syncthreads();  // every wave has read the list before the next one
-  }
-  rec.state = SEL_SLOW;
-  return rec;
 }
 
 // The block's examples in order (one workgroup of G threads, all of which
@@ -450,15 +163,16 @@ __device__ __forceinline__ SelectRecord<R> epoch_select(const D (&w)[PF], int mp
 // reads are the ones it wrote).  The block's delta rows live in LDS where
 // kEpochBlock rows always fit (DL), else in Delta (nb x m), which holds them
 // for the rank update in any case.  Gm: nb x nb Gram matrix.  gdummy: G
-// words of global memory, the threads' sinks for stores past m.  C: the
-// thresholds' column has G C words (C = 0: m).  PF > 0 (m <= G PF):
+// words of global memory, the threads' sinks for stores past m.  C, KM: the
+// register form of the simplex / knapsack thresholds for m - 1 <= G C values
+// (C = 0: the sorted-column form only) and k <= KM.  PF > 0 (m <= G PF):
 // each thread keeps its entries of the example's vector, of a_i and of S_k
 // in registers, the next example's a_i and S_k loaded while this one runs;
 // PF = 0 keeps the vector in LDS and reads a_i and S_k as it goes.  GV
 // (PF = 0, rows beyond the LDS): the vector, the thresholds' column and the
 // labels live in gv (global memory, the workspace; L2-resident at the sizes
 // where LDS ends), the same code reading them there.
-template <class D, class R, int FK, int C, int PF, bool GV = false>
+template <class D, class R, int FK, int C, int KM, int PF, bool GV = false>
 __global__ void __launch_bounds__(kEpochThreads)
 epoch_block_kernel(const D* __restrict__ S, const D* __restrict__ Gm,
                    const int64_t* __restrict__ order, int64_t q0, int64_t n, int nb,
@@ -469,8 +183,6 @@ epoch_block_kernel(const D* __restrict__ S, const D* __restrict__ Gm,
   constexpr int G = kEpochThreads;
   constexpr int PQ = PF > 0 ? PF : 1;
   constexpr bool DL = epoch_delta_in_lds<D>(PF);
-  constexpr bool SEL = FK == kFamHinge && PF > 0;  // the hinges by selection
-  constexpr bool SIDE = SEL && DL && PF > 1;
   static_assert(!GV || (PF == 0 && !DL), "global vectors for the PF = 0 form");
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const int cw = epoch_column_words(m, C);
@@ -484,6 +196,7 @@ epoch_block_kernel(const D* __restrict__ S, const D* __restrict__ Gm,
   int* const lab = GV ? reinterpret_cast<int*>(cb + cw)
                       : reinterpret_cast<int*>(dummy + G + (DL ? epoch_dx_words(m, PF) : 0));
   __shared__ R sh_t, sh_lo, sh_hi;
+  __shared__ int sh_slow;
   __shared__ D sh_vy;
   __shared__ D g_all[kEpochBlock * kEpochBlock];
   __shared__ D sh_norm[kEpochBlock];
@@ -491,21 +204,6 @@ epoch_block_kernel(const D* __restrict__ S, const D* __restrict__ Gm,
   __shared__ int sh_y[kEpochBlock];   // multiclass: the label; multilabel: the label count
   __shared__ int64_t sh_off[kEpochBlock];
   __shared__ int sh_badex;
-  // The hinges by selection (PF > 0): the threads' maxima, the sorted list
-  // and its prefix sums, the waves' candidate counts, the label's old entry.
-  __shared__ D sh_parts[SEL ? kEpochThreads : 1];
-  __shared__ D sh_list[SEL ? kSelectMax : 1];
-  __shared__ double sh_ps[SEL ? kSelectMax + 2 : 1];
-  __shared__ int sh_counts[SEL ? 2 * kEpochThreads / 64 : 1];
-  __shared__ D sh_ay;
-  __shared__ EpochSums<R> sh_xs[SEL ? 2 * kEpochThreads / 64 : 1];
-  // The hinges' coefficients per example, and the waves' sums of an example
-  // (one of two sets in turn, so that an exchange is one barrier).
-  __shared__ R sh_rho[SEL ? kEpochBlock : 1];
-  __shared__ D sh_pa[SEL ? kEpochBlock : 1];
-  __shared__ R sh_sum[2][SEL ? kEpochThreads / 64 : 1];
-  __shared__ D sh_asum[2][SEL ? kEpochThreads / 64 : 1];
-  const int dstride = (DL && SIDE) ? (m + 3) & ~3 : m;  // of the delta rows
   const int tid = static_cast<int>(threadIdx.x);
   const int lane = tid & 63;
   D* const ld = dummy + tid;   // LDS sink
@@ -547,14 +245,8 @@ epoch_block_kernel(const D* __restrict__ S, const D* __restrict__ Gm,
       }
     }
     sh_i[tid] = i;
-    const D norm2 = norms[i];
-    sh_norm[tid] = norm2;
+    sh_norm[tid] = norms[i];
     sh_y[tid] = static_cast<int>(yl);
-    if constexpr (SEL) {
-      const R rho = smooth ? static_cast<R>(norm2) / (static_cast<R>(norm2) + gamma / c) : R(1);
-      sh_rho[tid] = rho;
-      sh_pa[tid] = smooth ? static_cast<D>(rho) / norm2 : D(1) / norm2;
-    }
   }
   for (int e = tid; e < nb * nb; e += G) g_all[e] = Gm[e];
   __syncthreads();
@@ -562,18 +254,13 @@ epoch_block_kernel(const D* __restrict__ S, const D* __restrict__ Gm,
   // one example ahead and copied at the top of its step, where nothing newer
   // is in flight (so the wait for them waits for nothing else).
   D acur[PQ], anext[PQ], scur[PQ], snext[PQ], vr[PQ];
-  // The thread's columns of a row in global memory (the last one past m).
-  auto load_row = [&](const D* row, D (&x)[PQ]) {
-    if (SIDE && PF * tid + PF <= m) {
-#pragma unroll
-      for (int q = 0; q < PF; ++q) x[q] = row[PF * tid + q];
-    } else {
-      for_cols<PF, SIDE>(tid, m, [&](int j, int q, bool ok) { x[q] = row[ok ? j : m - 1]; });
-    }
-  };
   if constexpr (PF > 0) {
-    load_row(A + sh_i[0] * m, anext);
-    load_row(S, snext);
+    const D* a0 = A + sh_i[0] * m;
+    for_cols<PF>(tid, m, [&](int j, int q, bool ok) {
+      const int jc = ok ? j : m - 1;
+      anext[q] = a0[jc];
+      snext[q] = S[jc];
+    });
   }
   // The example's vector entry of slot (j, q): registers or LDS.
   auto getv = [&](int j, int q) -> D {
@@ -602,8 +289,13 @@ epoch_block_kernel(const D* __restrict__ S, const D* __restrict__ Gm,
       // The next example's a as A holds it now (replaced below when it is
       // this example, the only one whose update is still to come).
       if (has_next) {
-        load_row(A + sh_i[k + 1] * m, anext);
-        load_row(srow + m, snext);
+        const D* an = A + sh_i[k + 1] * m;
+        const D* sn = srow + m;
+        for_cols<PF>(tid, m, [&](int j, int q, bool ok) {
+          const int jc = ok ? j : m - 1;
+          anext[q] = an[jc];
+          snext[q] = sn[jc];
+        });
       }
     }
     if (ml && y > 0) {
@@ -620,17 +312,13 @@ epoch_block_kernel(const D* __restrict__ S, const D* __restrict__ Gm,
       }
     }
     if (!(norm2 > D(0)) || (ml && y == 0)) {  // update.h:62: the example changes nothing
-      for_cols<PF, SIDE>(tid, m, [&](int j, int q, bool ok) { *(ok ? drow + j : gd) = D(0); });
+      for_cols<PF>(tid, m, [&](int j, int q, bool ok) { *(ok ? drow + j : gd) = D(0); });
       continue;
     }
     // 1. The vector to project: axpby(pa, scores, pb, a_old).
     R rho = R(1);
     D pa = D(1), pb = -norm2;  // the entropic objectives
-    if constexpr (SEL) {
-      rho = sh_rho[k];
-      pa = sh_pa[k];
-      pb = smooth ? -static_cast<D>(rho) : D(-1);
-    } else if (hinge) {
+    if (hinge) {
       rho = smooth ? static_cast<R>(norm2) / (static_cast<R>(norm2) + gamma / c) : R(1);
       pa = smooth ? static_cast<D>(rho) / norm2 : D(1) / norm2;
       pb = smooth ? -static_cast<D>(rho) : D(-1);
@@ -667,31 +355,21 @@ epoch_block_kernel(const D* __restrict__ S, const D* __restrict__ Gm,
         D dv[kFixRows][PQ];
 #pragma unroll
         for (int b = 0; b < kFixRows; ++b) {
-          const D* drr = Dx + static_cast<int64_t>(rr[b]) * dstride;
-          if constexpr (DL && SIDE) {
-            typedef D row_word __attribute__((ext_vector_type(PF)));
-            const row_word x = *reinterpret_cast<const row_word*>(drr + PF * tid);
-#pragma unroll
-            for (int q = 0; q < PF; ++q) dv[b][q] = x[q];
-          } else if constexpr (DL) {
-            for_cols<PF, SIDE>(tid, m, [&](int j, int q, bool ok) { dv[b][q] = drr[j]; });
-          } else {
-            load_row(drr, dv[b]);
-          }
+          const D* drr = Dx + static_cast<int64_t>(rr[b]) * m;
+          for_cols<PF>(tid, m, [&](int j, int q, bool ok) {
+            dv[b][q] = drr[(DL || ok) ? j : m - 1];
+          });
         }
 #pragma unroll
         for (int b = 0; b < kFixRows; ++b) {
           if (base + b < nrows) {
 #pragma unroll
-            for (int q = 0; q < PF; ++q) {
-              if constexpr (sizeof(D) == 4) scur[q] = fma(-g[b], dv[b][q], scur[q]);
-              else scur[q] -= g[b] * dv[b][q];
-            }
+            for (int q = 0; q < PF; ++q) scur[q] -= g[b] * dv[b][q];
           }
         }
       }
     }
-    for_cols<PF, SIDE>(tid, m, [&](int j, int q, bool ok) {
+    for_cols<PF>(tid, m, [&](int j, int q, bool ok) {
       D sc, ao;
       if constexpr (PF > 0) {
         sc = scur[q];
@@ -704,29 +382,15 @@ epoch_block_kernel(const D* __restrict__ S, const D* __restrict__ Gm,
       }
       const D x = pa * sc + pb * ao;
       setv(j, q, x);
-      if constexpr (PF > 0 && !SEL) *((ok && j == y) ? &sh_vy : ld) = x;
+      if constexpr (PF > 0) *((ok && j == y) ? &sh_vy : ld) = x;
     });
-    if constexpr (SEL) {
-      D part = -num<D>::inf();
-      for_cols<PF, SIDE>(tid, m, [&](int j, int q, bool ok) {
-        part = (ok && j != y && vr[q] > part) ? vr[q] : part;
-      });
-      sh_parts[tid] = part;
-      for_cols<PF, SIDE>(tid, m, [&](int j, int q, bool ok) {
-        if (j == y) {
-          sh_vy = vr[q];
-          sh_ay = acur[q];
-        }
-      });
-    }
     __syncthreads();
     if (ml && sh_badex == k) {  // labels not valid: the example is skipped
-      for_cols<PF, SIDE>(tid, m, [&](int j, int q, bool ok) { *(ok ? drow + j : gd) = D(0); });
+      for_cols<PF>(tid, m, [&](int j, int q, bool ok) { *(ok ? drow + j : gd) = D(0); });
       __syncthreads();
       continue;
     }
     const D vy = PF > 0 ? sh_vy : v[y];
-    const D ay_old = SEL ? sh_ay : D(0);
     if constexpr (ml) {
       // The labels first (output.h:121-164): label r of the example (the
       // r-th smallest) to row r, the other rows after them in index order;
@@ -744,7 +408,7 @@ epoch_block_kernel(const D* __restrict__ S, const D* __restrict__ Gm,
       };
       constexpr bool ent = FK == kFamMlEnt;
       const D half = pa / D(2);
-      for_cols<PF, SIDE>(tid, m, [&](int j, int q, bool ok) {
+      for_cols<PF>(tid, m, [&](int j, int q, bool ok) {
         bool is_lab;
         const int r = rank_of(j, is_lab);
         const D x = getv(j, q);
@@ -760,7 +424,7 @@ epoch_block_kernel(const D* __restrict__ S, const D* __restrict__ Gm,
         const D map_a = D(1) / static_cast<D>(alpha);
         const D ta = static_cast<D>(t), tb = static_cast<D>(t + c2);
         const D na = static_cast<D>(-c), nbias = static_cast<D>(c / static_cast<R>(nl));
-        for_cols<PF, SIDE>(tid, m, [&](int j, int q, bool ok) {
+        for_cols<PF>(tid, m, [&](int j, int q, bool ok) {
           bool is_lab;
           rank_of(j, is_lab);
           const D x = clamp_ref(map_a * lambert_w_exp_nb(getv(j, q) - (is_lab ? ta : tb)), D(0),
@@ -796,7 +460,7 @@ epoch_block_kernel(const D* __restrict__ S, const D* __restrict__ Gm,
           tb = static_cast<D>(th.t2);
         }
         const D hc = static_cast<D>(c);
-        for_cols<PF, SIDE>(tid, m, [&](int j, int q, bool ok) {
+        for_cols<PF>(tid, m, [&](int j, int q, bool ok) {
           bool is_lab;
           rank_of(j, is_lab);
           const D x = getv(j, q);
@@ -805,7 +469,7 @@ epoch_block_kernel(const D* __restrict__ S, const D* __restrict__ Gm,
       }
     } else if constexpr (FK == kFamEnt) {
       // prox_two_entropy over (label | the rest), alpha = c norm2
-      for_cols<PF, SIDE>(tid, m, [&](int j, int q, bool ok) {
+      for_cols<PF>(tid, m, [&](int j, int q, bool ok) {
         *(ok ? cb + (j == y ? 0 : (j < y ? j + 1 : j)) : ld) = getv(j, q);
       });
       __syncthreads();
@@ -815,125 +479,15 @@ epoch_block_kernel(const D* __restrict__ S, const D* __restrict__ Gm,
       const D map_a = D(1) / static_cast<D>(alpha);
       const D ta = static_cast<D>(t), tb = static_cast<D>(t + c2);
       const D na = static_cast<D>(-c), nbias = static_cast<D>(c / R(1));
-      for_cols<PF, SIDE>(tid, m, [&](int j, int q, bool ok) {
+      for_cols<PF>(tid, m, [&](int j, int q, bool ok) {
         const D x = clamp_ref(map_a * lambert_w_exp_nb(getv(j, q) - (j == y ? ta : tb)), D(0), D(1));
         setv(j, q, (j == y) ? na * x + nbias : na * x);
       });
-    } else if constexpr (SEL) {
-      // The off-label entries shifted by (pa - v_y); the label's slot holds
-      // none.
-      const D shift = pa - vy;
-      D w[PF];
-      for_cols<PF, SIDE>(tid, m, [&](int j, int q, bool ok) {
-        w[q] = (ok && j != y) ? vr[q] + shift : -num<D>::inf();
-      });
-      const int mp = m - 1;
-      ProxParamsT<R> pp;
-      pp.lo = R(0);
-      pp.hi = knap_hi;
-      pp.rhs = c;
-      pp.rho = rho;
-      pp.k = ob.k;
-      pp.rhs_k = c / static_cast<R>(ob.k);
-      pp.op = op;
-      pp.p = 0;
-      SelectRecord<R> rec;
-      rec.state = SEL_SLOW;
-      // (one of the two counter sets per example in turn)
-      if (mp <= kSelectMax || ob.k < kSearchRankLast)
-        rec = epoch_select<PF, D, R>(w, mp, shift, pp, sh_parts, cb, sh_list, sh_ps,
-                                     sh_counts + (k & 1) * (G / 64), sh_xs);
-      if (rec.state != SEL_DONE) {
-        // The whole column sorted in LDS, compacted (any order).
-        __syncthreads();
-        for_cols<PF, SIDE>(tid, m, [&](int j, int q, bool ok) {
-          *((ok && j != y) ? cb + (j < y ? j : j - 1) : ld) = w[q];
-        });
-        __syncthreads();
-        sort_desc_unpadded(cb, mp);
-        if (tid < 64) {
-          R t, lo, hi;
-          int branch, n_hi, n_mid;  // (not used by the epoch)
-          thresholds_sorted<D, R>(cb, mp, op, R(0), knap_hi, c, rho, ob.k, t, lo, hi, branch, n_hi,
-                                  n_mid);
-          if (lane == 0) {
-            sh_t = t;
-            sh_hi = hi;
-          }
-        }
-        __syncthreads();
-        rec.t = sh_t;
-        rec.hi = sh_hi;
-      }
-      // Clamp, recover the variables (the label's entry from the sum, the
-      // others negated), a_old - a_new and its 1-norm: the clamped entries'
-      // sum and the norm over them in one exchange.
-      const D t = static_cast<D>(rec.t), hi = static_cast<D>(rec.hi);
-      R sum = 0;
-      D asum = 0;
-      for_cols<PF, SIDE>(tid, m, [&](int j, int q, bool ok) {
-        const bool off = ok && j != y;
-        const D x = clamp_ref(w[q] - t, D(0), hi);
-        sum += off ? static_cast<R>(x) : R(0);
-        asum += off ? fabs(acur[q] + x) : D(0);
-        vr[q] = -x;
-      });
-      sum = wave_total(sum);
-      asum = wave_total(asum);
-      if (lane == 0) {
-        sh_sum[k & 1][tid >> 6] = sum;
-        sh_asum[k & 1][tid >> 6] = asum;
-      }
-      __syncthreads();
-      sum = sh_sum[k & 1][0];
-      asum = sh_asum[k & 1][0];
-#pragma unroll
-      for (int i = 1; i < G / 64; ++i) {
-        sum += sh_sum[k & 1][i];
-        asum += sh_asum[k & 1][i];
-      }
-      const D ay = static_cast<D>(dmin(c, sum));
-      asum += fabs(ay_old - ay);
-      const bool moves = asum > num<D>::eps() || ob.kernel;
-      D dl[PF];
-      for_cols<PF, SIDE>(tid, m, [&](int j, int q, bool ok) {
-        vr[q] = (j == y) ? ay : vr[q];
-        dl[q] = acur[q] - vr[q];
-      });
-      if constexpr (DL && SIDE) {
-        if (PF * tid < m) {  // (a row's padding holds the tail past m)
-          typedef D row_word __attribute__((ext_vector_type(PF)));
-          row_word x;
-#pragma unroll
-          for (int q = 0; q < PF; ++q) x[q] = dl[q];
-          *reinterpret_cast<row_word*>(Dx + static_cast<int64_t>(k) * dstride + PF * tid) = x;
-        }
-      }
-      if (SIDE && PF * tid + PF <= m) {
-#pragma unroll
-        for (int q = 0; q < PF; ++q) drow[PF * tid + q] = moves ? dl[q] : D(0);
-#pragma unroll
-        for (int q = 0; q < PF; ++q) arow[PF * tid + q] = vr[q];
-      } else {
-        for_cols<PF, SIDE>(tid, m, [&](int j, int q, bool ok) {
-          *(ok ? drow + j : gd) = moves ? dl[q] : D(0);
-          *(ok ? arow + j : gd) = vr[q];
-          if constexpr (DL && !SIDE) *(ok ? Dx + static_cast<int64_t>(k) * dstride + j : ld) = dl[q];
-        });
-      }
-      if (moves) changed |= 1u << k;  // the later examples' scores see this update
-      if (has_next && sh_i[k + 1] == i) {
-#pragma unroll
-        for (int q = 0; q < PF; ++q) anext[q] = vr[q];
-      }
-      // (the next example's writes of the shared entries are behind this
-      // example's exchange; its delta row is read by the threads that wrote it)
-      continue;
     } else {
       // The off-label entries shifted by (pa - v_y) (hinge) or -v_y (top-k
       // entropy), compacted into cb.
       const D shift = hinge ? pa - vy : -vy;
-      for_cols<PF, SIDE>(tid, m, [&](int j, int q, bool ok) {
+      for_cols<PF>(tid, m, [&](int j, int q, bool ok) {
         const bool off = j != y;
         const D x = getv(j, q) + shift;
         if (off) setv(j, q, x);
@@ -942,16 +496,58 @@ epoch_block_kernel(const D* __restrict__ S, const D* __restrict__ Gm,
       __syncthreads();
       const int mp = m - 1;
       if constexpr (hinge) {
-        sort_desc_unpadded(cb, mp);
-        if (tid < 64) {
-          R t, lo, hi;
-          int branch, n_hi, n_mid;  // (not used by the epoch)
-          thresholds_sorted<D, R>(cb, mp, op, R(0), knap_hi, c, rho, ob.k, t, lo, hi, branch, n_hi,
-                                  n_mid);
-          if (lane == 0) {
-            sh_t = t;
-            sh_lo = lo;
-            sh_hi = hi;
+        bool sorted_form = true;
+        if constexpr (C > 0) {
+          // The register form over the whole workgroup (slot c of thread g
+          // = entry g + G c), which defers to the sorted form only where the
+          // reference's biased cone search is needed
+          // (topk_simplex_biased.h:57-66).
+          D vq[C];
+          const int nvalid = (mp - tid + G - 1) / G;
+#pragma unroll
+          for (int q = 0; q < C; ++q) {
+            const D x = cb[tid + G * q];
+            vq[q] = (q < nvalid) ? x : -num<D>::inf();
+          }
+          ProxParamsT<R> pp;
+          pp.lo = R(0);
+          pp.hi = knap_hi;
+          pp.rhs = c;
+          pp.rho = rho;
+          pp.k = ob.k;
+          pp.rhs_k = (ob.k > 0) ? c / static_cast<R>(ob.k) : R(0);
+          pp.op = op;
+          pp.p = 0;
+          const ColThr<R> th = simplex
+              ? topk_family<G, C, KM, D, R, false>(vq, mp, nvalid, pp, cb, ld)
+              : knap_family<G, C, D, R>(vq, mp, nvalid, pp);
+          if (tid == 0) {
+            sh_slow = th.slow ? 1 : 0;
+            sh_t = th.t;
+            sh_lo = th.lo;
+            sh_hi = th.hi;
+          }
+          __syncthreads();
+          sorted_form = sh_slow != 0;
+          if (sorted_form) {  // cb served as scratch: compact it again
+            for_cols<PF>(tid, m, [&](int j, int q, bool ok) {
+              *((ok && j != y) ? cb + (j < y ? j : j - 1) : ld) = getv(j, q);
+            });
+            __syncthreads();
+          }
+        }
+        if (sorted_form) {
+          sort_desc_unpadded(cb, mp);
+          if (tid < 64) {
+            R t, lo, hi;
+            int branch, n_hi, n_mid;  // (not used by the epoch)
+            thresholds_sorted<D, R>(cb, mp, op, R(0), knap_hi, c, rho, ob.k, t, lo, hi, branch,
+                                    n_hi, n_mid);
+            if (lane == 0) {
+              sh_t = t;
+              sh_lo = lo;
+              sh_hi = hi;
+            }
           }
         }
       } else {  // prox_topk_entropy_biased, alpha = c norm2
@@ -967,7 +563,7 @@ epoch_block_kernel(const D* __restrict__ S, const D* __restrict__ Gm,
       const D t = static_cast<D>(sh_t), lo = static_cast<D>(sh_lo), hi = static_cast<D>(sh_hi);
       const D map_a = hinge ? D(1) : D(1) / static_cast<D>(c * static_cast<R>(norm2));
       R part = 0;
-      for_cols<PF, SIDE>(tid, m, [&](int j, int q, bool ok) {
+      for_cols<PF>(tid, m, [&](int j, int q, bool ok) {
         const bool off = j != y;
         const D x0 = getv(j, q);
         const D x = hinge ? clamp_ref(x0 - t, lo, hi)
@@ -980,13 +576,13 @@ epoch_block_kernel(const D* __restrict__ S, const D* __restrict__ Gm,
       // negated (and scaled by c for the top-k entropy).
       const D scale = hinge ? D(-1) : static_cast<D>(-c);
       const D ay = hinge ? static_cast<D>(dmin(c, sum)) : static_cast<D>(c * dmin(R(1), sum));
-      for_cols<PF, SIDE>(tid, m, [&](int j, int q, bool ok) {
+      for_cols<PF>(tid, m, [&](int j, int q, bool ok) {
         setv(j, q, (j == y) ? ay : getv(j, q) * scale);
       });
     }
     // a_old - a_new (sdca_blas_axpy with -1), its 1-norm, a_i <- a_new.
     D part = 0;
-    for_cols<PF, SIDE>(tid, m, [&](int j, int q, bool ok) {
+    for_cols<PF>(tid, m, [&](int j, int q, bool ok) {
       const D an = getv(j, q);
       const D dl = (PF > 0 ? acur[q] : arow[j]) + D(-1) * an;
       *(ok ? drow + j : gd) = dl;
@@ -998,7 +594,7 @@ epoch_block_kernel(const D* __restrict__ S, const D* __restrict__ Gm,
     if (asum > num<D>::eps() || ob.kernel) {
       changed |= 1u << k;  // the later examples' scores see this update
     } else {
-      for_cols<PF, SIDE>(tid, m, [&](int j, int q, bool ok) { *(ok ? drow + j : gd) = D(0); });
+      for_cols<PF>(tid, m, [&](int j, int q, bool ok) { *(ok ? drow + j : gd) = D(0); });
     }
     if constexpr (PF > 0) {
       if (has_next && sh_i[k + 1] == i) {
@@ -1275,7 +871,7 @@ __host__ inline size_t block_lds_bytes(size_t es, int m, int C, int PF, bool del
   return lds;
 }
 
-template <class D, class R, int FK, int C, int PF>
+template <class D, class R, int FK, int C, int KM, int PF>
 hipError_t launch_block(const D* S, const D* Gm, int64_t q0, int nb, const D* norms,
                         const EpochLaunch& a, D* Delta, D* gdummy, const EpochObj& ob, int* bad,
                         D* gv) {
@@ -1286,7 +882,7 @@ hipError_t launch_block(const D* S, const D* Gm, int64_t q0, int nb, const D* no
     // Rows beyond the LDS: the PF = 0 form with its vectors in gv (the
     // workspace holds epoch_gv_words(m) words there).
     if constexpr (PF == 0 && C == 0) {
-      hipLaunchKernelGGL((epoch_block_kernel<D, R, FK, C, PF, true>), dim3(1),
+      hipLaunchKernelGGL((epoch_block_kernel<D, R, FK, C, KM, PF, true>), dim3(1),
                          dim3(kEpochThreads), kEpochThreads * sizeof(D), a.stream, S, Gm,
                          a.order, q0, a.n, nb, norms, a.labels, a.offsets, static_cast<D*>(a.A),
                          Delta, gdummy, ob, m, bad, gv);
@@ -1295,29 +891,29 @@ hipError_t launch_block(const D* S, const D* Gm, int64_t q0, int nb, const D* no
       return hipErrorInvalidValue;
     }
   }
-  hipLaunchKernelGGL((epoch_block_kernel<D, R, FK, C, PF>), dim3(1), dim3(kEpochThreads), lds,
+  hipLaunchKernelGGL((epoch_block_kernel<D, R, FK, C, KM, PF>), dim3(1), dim3(kEpochThreads), lds,
                      a.stream, S, Gm, a.order, q0, a.n, nb, norms, a.labels, a.offsets,
                      static_cast<D*>(a.A), Delta, gdummy, ob, m, bad, gv);
   return hipGetLastError();
 }
 
 // The block kernel for the objective's family, m and k: register slots per
-// thread PF from m (m <= 256, 1024, 2048), and C = PF for the multiclass
-// hinges (the selection's candidates take the column's G C words) and for
-// the register form of the multilabel hinges' two-block simplex.
+// thread PF from m (m <= 256, 1024, 2048), and the register forms (C = PF)
+// of the multiclass hinges' simplex / knapsack thresholds (k <= 8 for the
+// simplex) and of the multilabel hinges' two-block simplex.
 template <class D, class R>
 hipError_t launch_block_for(const D* S, const D* Gm, int64_t q0, int nb, const D* norms,
                             const EpochLaunch& a, D* Delta, D* gdummy, const EpochObj& ob,
                             int* bad, D* gv) {
   const int64_t m = a.m;
   const int pf = m <= 256 ? 1 : m <= 1024 ? 4 : m <= 2048 ? 8 : 0;
-#define SDCA_EPOCH_BLOCK(FK, C, PF) \
-  launch_block<D, R, FK, C, PF>(S, Gm, q0, nb, norms, a, Delta, gdummy, ob, bad, gv)
+#define SDCA_EPOCH_BLOCK(FK, C, KM, PF) \
+  launch_block<D, R, FK, C, KM, PF>(S, Gm, q0, nb, norms, a, Delta, gdummy, ob, bad, gv)
   // Families without a register form: one variant per PF.
 #define SDCA_EPOCH_BY_PF(FK)                                      \
-  (pf == 0 ? SDCA_EPOCH_BLOCK(FK, 0, 0)                        \
-           : pf == 1 ? SDCA_EPOCH_BLOCK(FK, 0, 1)              \
-                     : pf == 4 ? SDCA_EPOCH_BLOCK(FK, 0, 4) : SDCA_EPOCH_BLOCK(FK, 0, 8))
+  (pf == 0 ? SDCA_EPOCH_BLOCK(FK, 0, 5, 0)                        \
+           : pf == 1 ? SDCA_EPOCH_BLOCK(FK, 0, 5, 1)              \
+                     : pf == 4 ? SDCA_EPOCH_BLOCK(FK, 0, 5, 4) : SDCA_EPOCH_BLOCK(FK, 0, 5, 8))
   hipError_t e;
   switch (a.kind) {
     case SDCA_OBJ_ENTROPY:
@@ -1331,16 +927,25 @@ hipError_t launch_block_for(const D* S, const D* Gm, int64_t q0, int nb, const D
       break;
     case SDCA_OBJ_MULTILABEL_HINGE:
     case SDCA_OBJ_MULTILABEL_HINGE_SMOOTH:
-      e = pf == 0 ? SDCA_EPOCH_BLOCK(kFamMlHinge, 0, 0)
-                  : pf == 1 ? SDCA_EPOCH_BLOCK(kFamMlHinge, 1, 1)
-                            : pf == 4 ? SDCA_EPOCH_BLOCK(kFamMlHinge, 4, 4)
-                                      : SDCA_EPOCH_BLOCK(kFamMlHinge, 8, 8);
+      e = pf == 0 ? SDCA_EPOCH_BLOCK(kFamMlHinge, 0, 5, 0)
+                  : pf == 1 ? SDCA_EPOCH_BLOCK(kFamMlHinge, 1, 5, 1)
+                            : pf == 4 ? SDCA_EPOCH_BLOCK(kFamMlHinge, 4, 5, 4)
+                                      : SDCA_EPOCH_BLOCK(kFamMlHinge, 8, 5, 8);
       break;
-    default:
-      e = pf == 0 ? SDCA_EPOCH_BLOCK(kFamHinge, 0, 0)
-                  : pf == 1 ? SDCA_EPOCH_BLOCK(kFamHinge, 1, 1)
-                            : pf == 4 ? SDCA_EPOCH_BLOCK(kFamHinge, 4, 4)
-                                      : SDCA_EPOCH_BLOCK(kFamHinge, 8, 8);
+    default: {
+      const bool simplex = a.kind == SDCA_OBJ_HINGE_TOPK || a.kind == SDCA_OBJ_HINGE_TOPK_SMOOTH;
+      if (pf == 0 || (simplex && a.k > 8)) {
+        e = SDCA_EPOCH_BY_PF(kFamHinge);
+      } else if (!simplex || a.k <= 5) {
+        e = pf == 1 ? SDCA_EPOCH_BLOCK(kFamHinge, 1, 5, 1)
+                    : pf == 4 ? SDCA_EPOCH_BLOCK(kFamHinge, 4, 5, 4)
+                              : SDCA_EPOCH_BLOCK(kFamHinge, 8, 5, 8);
+      } else {
+        e = pf == 1 ? SDCA_EPOCH_BLOCK(kFamHinge, 1, 8, 1)
+                    : pf == 4 ? SDCA_EPOCH_BLOCK(kFamHinge, 4, 8, 4)
+                              : SDCA_EPOCH_BLOCK(kFamHinge, 8, 8, 8);
+      }
+    }
   }
 #undef SDCA_EPOCH_BY_PF
 #undef SDCA_EPOCH_BLOCK

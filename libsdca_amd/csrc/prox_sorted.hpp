@@ -147,8 +147,8 @@ __device__ inline bool wave_first_accept(int& u_found, R& t, R& hi, int& e) {
 // a step at whose end t has reached the next value (less a bound of the
 // sums' rounding); once t stays above every value still to come, no later M
 // can be accepted.  Bound by the chain of additions.  A first epoch at m =
-// 1000, d = 4096, most of whose searches end with about 900 values in M:
-// 50 us per example with every trial formed, 30 so.
+// 1000, d = 4096, n = 20,000, most of whose searches end with about 900
+// values in M: 786 ms with every trial formed, 427 so, the same bits.
 //
 // s may hold only the cnt largest of the m values, the others at most `cut`:
 // false where a search may go on past them.

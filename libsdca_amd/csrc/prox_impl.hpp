@@ -338,9 +338,12 @@ __device__ inline R knapsack_biased_regs(const D (&v)[C], int m, R total, R lo, 
 
 // ---------------------------------------------------------------------------
 // Knapsack family: knapsack_eq (knapsack_eq.h:25-109) and knapsack_le
-// (knapsack_le.h:17-44).
+// (knapsack_le.h:17-44).  MAX_START: the start from the bound max - rhs below
+// (the prox kernels).  The SDCA epoch goes without it: its hinge takes that
+// start at k = 1 only, and carried its exchange buffer (1 KiB of LDS), up to
+// nine registers and the spilled scalars of its branch for every other k.
 // ---------------------------------------------------------------------------
-template <int G, int C, class D, class R>
+template <int G, int C, class D, class R, bool MAX_START = true>
 __device__ inline ColThr<R> knap_family(const D (&v)[C], int m, int nvalid,
                                         const ProxParamsT<R>& pp) {
   const R lo = pp.lo, hi = pp.hi, rhs = pp.rhs;
@@ -374,7 +377,7 @@ __device__ inline ColThr<R> knap_family(const D (&v)[C], int m, int nvalid,
   // float column: there the rounding of the fixing's numerator (sums of
   // thousands over a dozen free values) decides which values near t are free,
   // and it takes the sorted column's steps from the mean on.
-  const bool from_max = lo == R(0) && hi >= rhs && sizeof(S) == sizeof(R);
+  const bool from_max = MAX_START && sizeof(S) == sizeof(R) && lo == R(0) && hi >= rhs;
   if (from_max) {
     R mx = -num<R>::inf(), sum = 0;
 #pragma unroll

@@ -149,19 +149,16 @@ __device__ inline bool wave_first_accept(int& u_found, R& t, R& hi, int& e) {
 // can be accepted.  Bound by the chain of additions.  A first epoch at m =
 // 1000, d = 4096, n = 20,000, most of whose searches end with about 900
 // values in M: 786 ms with every trial formed, 427 so, the same bits.
-//
-// s may hold only the cnt largest of the m values, the others at most `cut`:
-// false where a search may go on past them.
 constexpr int kConeStep = 16;
 template <class D, class R>
-__device__ bool cone_search_sorted(const D* s, int cnt, int m, R cut, int k, R rho, R& t_out,
-                                   R& hi_out, int& branch, int& n_hi, int& n_mid) {
+__device__ void cone_search_sorted(const D* s, int m, int k, R rho, R& t_out, R& hi_out,
+                                   int& branch, int& n_hi, int& n_mid) {
   const R eps = R(16) * num<R>::eps();
   // How far the sums' rounding can move t: m additions, relative to the
   // largest value.
-  const R far = dmax(fabs(static_cast<R>(s[0])), fabs(static_cast<R>(s[cnt - 1])));
+  const R far = dmax(fabs(static_cast<R>(s[0])), fabs(static_cast<R>(s[m - 1])));
   const R slack = R(2) * eps + R(8) * num<R>::eps() * static_cast<R>(m + k) * far;
-  int found = INT_MAX, fe = 0, over = INT_MAX;
+  int found = INT_MAX, fe = 0;
   R ft = 0, fh = 0;
   const int lane = static_cast<int>(threadIdx.x) & 63;
   for (int base = 0; base <= k; base += 64) {
@@ -182,7 +179,7 @@ __device__ bool cone_search_sorted(const D* s, int cnt, int m, R cut, int k, R r
     int ml = mf;
     while (__ballot(active)) {
       if (active) {
-        bool trial = ml + kConeStep >= cnt;
+        bool trial = ml + kConeStep >= m;
         if (!trial) {
           R sm = sum_m, ns = num_m_sum_u, dn = den;
 #pragma unroll
@@ -209,8 +206,7 @@ __device__ bool cone_search_sorted(const D* s, int cnt, int m, R cut, int k, R r
             const R hi = (num_m_sum_u + k_u * sum_m) / den;
             const R tt = hi + t;
             if (max_m - eps <= tt && tt <= min_u + eps) {
-              if (t <= min_m + eps &&
-                  (ml == m || (ml < cnt ? static_cast<R>(s[ml]) : cut) - eps <= t)) {
+              if (t <= min_m + eps && (ml == m || static_cast<R>(s[ml]) - eps <= t)) {
                 found = mf;
                 fe = ml;
                 ft = t;
@@ -223,12 +219,9 @@ __device__ bool cone_search_sorted(const D* s, int cnt, int m, R cut, int k, R r
               active = false;
               break;
             }
-            if (i == kConeStep - 1 || ml == cnt) {
-              const R next = ml < cnt ? static_cast<R>(s[ml]) : cut;
-              const R lead = num_u * sum_m - k_u_sum_u - next * den;
-              const bool ends = lead > slack * (den + static_cast<R>(m - ml) * num_u);
-              if (!ends && ml == cnt) over = mf;
-              if (ends || ml == cnt) {
+            if (i == kConeStep - 1) {
+              const R lead = num_u * sum_m - k_u_sum_u - static_cast<R>(s[ml]) * den;
+              if (lead > slack * (den + static_cast<R>(m - ml) * num_u)) {
                 active = false;
                 break;
               }
@@ -246,10 +239,8 @@ __device__ bool cone_search_sorted(const D* s, int cnt, int m, R cut, int k, R r
       const unsigned long long hit = __ballot(found != INT_MAX);
       if (hit && lane > __ffsll(hit) - 1) active = false;
     }
-    if (__ballot(found != INT_MAX || over != INT_MAX)) break;
+    if (__ballot(found != INT_MAX)) break;
   }
-  over = group_min<64>(over);
-  if (group_min<64>(found) > over) return false;
   if (wave_first_accept(found, ft, fh, fe)) {
     branch = SDCA_BRANCH_SCAN;
     n_hi = found;
@@ -261,7 +252,6 @@ __device__ bool cone_search_sorted(const D* s, int cnt, int m, R cut, int k, R r
   }
   t_out = ft;
   hi_out = fh;
-  return true;
 }
 
 // thresholds_knapsack_le_biased_search (knapsack_le_biased.h:10-92) on the
@@ -398,7 +388,7 @@ __device__ void thresholds_sorted(const D* s, int m, int op, R lo, R hi, R rhs, 
       n_hi = k;
       n_mid = 0;
     } else {
-      cone_search_sorted<D, R>(s, m, m, R(0), k, rho, t_out, hi_out, branch, n_hi, n_mid);
+      cone_search_sorted<D, R>(s, m, k, rho, t_out, hi_out, branch, n_hi, n_mid);
     }
     return;
   }
@@ -423,7 +413,7 @@ __device__ void thresholds_sorted(const D* s, int m, int op, R lo, R hi, R rhs, 
       lt = K * (st.sum_u + (K - num_u) * st.t) < rhs * (num_u + rho * K * K) - eps;
     }
     if (lt) {
-      cone_search_sorted<D, R>(s, m, m, R(0), k, rho, t_out, hi_out, branch, n_hi, n_mid);
+      cone_search_sorted<D, R>(s, m, k, rho, t_out, hi_out, branch, n_hi, n_mid);
       return;
     }
   }

@@ -453,8 +453,8 @@ prox_select_kernel(const D* __restrict__ in, D* __restrict__ out, int64_t m64, i
         }
       }
       if (lead)
-        thresholds_sorted<D, R>(whole, m, pp.op, pp.lo, pp.hi, pp.rhs, pp.rho, k, rec.t, lo, rec.hi,
-                                rec.branch, rec.n_hi, rec.n_mid);
+        thresholds_sorted<D, R, true>(whole, m, pp.op, pp.lo, pp.hi, pp.rhs, pp.rho, k, rec.t, lo,
+                                      rec.hi, rec.branch, rec.n_hi, rec.n_mid);
       if constexpr (BT > 64) {
         if (threadIdx.x == 0) rec_lds = rec;
         __syncthreads();

@@ -58,7 +58,10 @@ __device__ inline void wave_sort_desc(D (&x)[CC]) {
   wave_sort_from<2, CC>(x, static_cast<int>(threadIdx.x) & 63, net_inf(D(0)));
 }
 
-// Exclusive prefix sum over the wave (as wave_exclusive_scan_dpp).
+// Exclusive prefix sum over the wave: the inclusive one (as
+// wave_exclusive_scan_dpp) of the lane before.  (Not the inclusive sum less
+// the lane's own value: next to a value far below the others, a masked
+// class at -1e9 say, that would round the sum of the others away.)
 __device__ inline double wave_exclusive_scan(double x) {
   double incl = x;
   incl = dpp_add<0x111, 0xF, true>(incl);   // row_shr:1
@@ -67,7 +70,11 @@ __device__ inline double wave_exclusive_scan(double x) {
   incl = dpp_add<0x118, 0xF, true>(incl);   // row_shr:8
   incl = dpp_add<0x142, 0xA, false>(incl);  // row_bcast:15
   incl = dpp_add<0x143, 0xC, false>(incl);  // row_bcast:31
-  return incl - x;
+  const long long u = __double_as_longlong(incl);
+  const int lo = dpp_bits<0x138, 0xF, true>(static_cast<int>(u & 0xffffffffll));  // wave_shr:1
+  const int hi = dpp_bits<0x138, 0xF, true>(static_cast<int>(u >> 32));
+  return __longlong_as_double((static_cast<long long>(hi) << 32) |
+                              static_cast<long long>(static_cast<unsigned>(lo)));
 }
 
 // A wave's sorted values x (value l CC + c in slot c of lane l, -inf from
@@ -132,22 +139,26 @@ struct SelectRecord {
 // sorted list (every value above t is in it): rank r is above t where
 // f(a_r) < rhs and at hi where f(a_r - hi) <= rhs, one rank per lane, f from
 // the prefix sums and a binary search for the ranks at hi (or inside) at
-// that point.  The same eps as the fixing's (topk_sorted_root).  The
+// that point.  The same eps as the fixing's (topk_sorted_root).  No rank at
+// or below a_(k) - hi is above t (there the k largest alone give k hi); far
+// below, the rounding of the test's large terms could say otherwise.  The
 // threshold is formed from the direct sum over the free ranks; with none
 // free any t of [a_u, a_(u-1) - hi] is the same projection and the record
 // takes the middle.
 template <class D, class R>
-__device__ inline void list_knapsack(const D* list, const double* ps, int cnt, int m, D cut, R hi_r,
-                                     R rhs_r, R& t_out, int& u_out, int& e_out) {
+__device__ inline void list_knapsack(const D* list, const double* ps, int cnt, int m, D cut, int k,
+                                     R hi_r, R rhs_r, R& t_out, int& u_out, int& e_out) {
   const int lane = static_cast<int>(threadIdx.x) & 63;
   const double hi = static_cast<double>(hi_r), rhs = static_cast<double>(rhs_r);
   const double eps = static_cast<double>(num<R>::eps() * dmax(R(1), fabs(rhs_r)));
+  const double kth = static_cast<double>(list[k - 1]);
+  const double least = kth - hi - 16.0 * static_cast<double>(num<R>::eps()) * (fabs(kth) + hi);
   int e = 0, u = 0;
   for (int base = 0; base < cnt; base += 64) {
     const int r = base + lane;
     bool above = false, at_hi = false;
-    if (r < cnt) {
-      const double a = static_cast<double>(list[r]);
+    const double a = r < cnt ? static_cast<double>(list[r]) : -num<double>::inf();
+    if (a > least) {
       int b = 0, w = r;
       while (b < w) {  // ranks above a + hi
         const int mid = (b + w) >> 1;
@@ -293,7 +304,7 @@ __device__ inline SelectRecord<R> list_record(const D* list, const double* ps, i
       return rec;
     }
     int u, e;
-    list_knapsack<D, R>(list, ps, cnt, m, cut, pp.rhs_k, rhs, rec.t, u, e);
+    list_knapsack<D, R>(list, ps, cnt, m, cut, k, pp.rhs_k, rhs, rec.t, u, e);
     bool lt = false;
     if (!constant) {
       if (u == 0) {

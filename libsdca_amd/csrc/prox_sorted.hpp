@@ -317,8 +317,10 @@ __device__ void knapsack_le_biased_sorted(const D* s, int m, R lo, R hi, R rhs, 
 
 // The record of the column's threshold function, with its branch
 // (sdca_prox_branch) and sets: n_hi, n_mid are positions in the sorted
-// column.
-template <class D, class R>
+// column.  BOUNDED: the top-k simplex's knapsack runs over the values above
+// a_(k) - hi only, as the register kernel's does (topk_knapsack); the others
+// end at 0, and classes masked by very low values stay out of its sums.
+template <class D, class R, bool BOUNDED = false>
 __device__ void thresholds_sorted(const D* s, int m, int op, R lo, R hi, R rhs, R rho, int k,
                                   R& t_out, R& lo_out, R& hi_out, int& branch, int& n_hi,
                                   int& n_mid) {
@@ -401,7 +403,12 @@ __device__ void thresholds_sorted(const D* s, int m, int op, R lo, R hi, R rhs, 
     n_mid = 0;
     return;
   }
-  KnapState<R> st = knapsack_sorted<D, R>(s, m, R(0), rhs / K, rhs);
+  int mk = m;
+  if constexpr (BOUNDED) {
+    const R kth = static_cast<R>(s[k - 1]), hi_k = rhs / K;
+    mk = prefix_end<R>(s, k, m, kth - hi_k - R(16) * num<R>::eps() * (fabs(kth) + hi_k));
+  }
+  KnapState<R> st = knapsack_sorted<D, R>(s, mk, R(0), rhs / K, rhs);
   if (!constant) {
     // is_topk_simplex_lt (topk_simplex.h:9-27) / is_topk_simplex_biased_lt
     // (topk_simplex_biased.h:9-28); rho = 0 gives the former exactly.

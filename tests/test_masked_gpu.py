@@ -1,0 +1,63 @@
+"""Columns of the top-k operators whose masked classes are set to a very low
+value.  A masked class ends at 0 and takes no part in the others' thresholds,
+so the outputs are those of the column without it, which the CPU oracle
+computes in long double.  Sizes on every path: the register kernel and its
+deferred columns, the selection by wave and by workgroup, and its fallback to
+the sorted column (more values at the mask than its list holds)."""
+import numpy as np
+import pytest
+
+from tests.test_prox_gpu import F32, F64
+
+pytestmark = pytest.mark.gpu
+
+OPS = [("topk_simplex", dict(rhs=1.0)), ("topk_cone", dict()),
+       ("topk_simplex_biased", dict(rhs=1.0, rho=0.5)), ("topk_cone_biased", dict(rho=0.25))]
+
+
+def masked_columns(m, k, dtype, mask, seed):
+    """N(0,1) columns with one label, all but some classes masked: one class,
+    half of them, all but k + 1, k, k - 1, and all but the first 16 (which sit
+    in few of the parts whose maxima give the selection its cut)."""
+    rng = np.random.default_rng(seed)
+    cols, keeps = [], []
+    for kept in (m - 1, m // 2, k + 1, k, k - 1, None):
+        keep = np.zeros(m, bool)
+        if kept is None:
+            keep[:16] = True
+        else:
+            keep[rng.permutation(m)[:kept]] = True
+        x = (rng.standard_normal(m) * 0.7).astype(dtype)
+        x[rng.integers(0, m)] += 2
+        x[~keep] = mask
+        cols.append(x)
+        keeps.append(keep)
+    return np.stack(cols), keeps
+
+
+def check_masked(oracle, cuda, op, kw, m, k, dtype, mask):
+    import torch
+    import libsdca_amd as sd
+    from oracle import binding
+    x, keeps = masked_columns(m, k, dtype, mask, m + k)
+    got = sd.prox(op, torch.from_numpy(x).to(cuda), k=k, **kw).cpu().numpy()
+    # a threshold's rounding: 4 (m + k) u of values of unit size
+    tol = 4 * (m + k) * float(np.finfo(dtype).eps)
+    for j, keep in enumerate(keeps):
+        want = np.zeros((1, int(keep.sum())))
+        if want.shape[1] >= k:  # fewer than k classes left: the cone is {0}
+            want = x[j, keep].astype(np.float64)[None, :].copy()
+            oracle.prox(op, want, result=2, params=binding.make_params(k=k, **kw))
+        err = np.abs(got[j, keep] - want[0]).max(initial=0.0)
+        assert err <= tol, f"{op} m={m} k={k} column {j} ({int(keep.sum())} kept): error {err:.2e}"
+        assert (got[j, ~keep] == 0).all(), f"{op} m={m} k={k} column {j}: a masked class is not 0"
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("m,k", [(40, 3), (100, 8), (300, 20), (700, 3), (1025, 8), (1500, 5),
+                                 (2048, 3)])
+@pytest.mark.parametrize("op,kw", OPS)
+def test_masked_low(cuda, oracle, op, kw, m, k, dtype):
+    """Finite masks, down to the type's lowest value."""
+    for mask in (-1e9, -1e30, -np.finfo(dtype).max):
+        check_masked(oracle, cuda, op, kw, m, k, dtype, dtype(mask))

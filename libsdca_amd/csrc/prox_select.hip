@@ -105,8 +105,12 @@ prox_select_kernel(const D* __restrict__ in, D* __restrict__ out, int64_t m64, i
     int tid = select_lane<BT>();
     asm("" : "+v"(tid));
     D v[C];
+    // Neither +inf nor NaN.  A value of -inf is a masked class: it ends at 0
+    // and is left out like the padding.
     bool finite = true;
-    R mag = 0;  // sum |a_i|, for the test of a close call (kClose)
+    // sum |a_i|, for the test of a close call (kClose; infinite with a masked
+    // class, which makes every call a close one)
+    R mag = 0;
     if (vec) {
       constexpr int E = 16 / static_cast<int>(sizeof(D));
       typedef D word __attribute__((ext_vector_type(E)));
@@ -117,7 +121,7 @@ prox_select_kernel(const D* __restrict__ in, D* __restrict__ out, int64_t m64, i
         const word x = *reinterpret_cast<const word*>(col + (ok ? i : 0));
 #pragma unroll
         for (int l = 0; l < E; ++l) {
-          finite = finite && fabs(x[l]) < num<D>::inf();
+          finite = finite && x[l] < num<D>::inf();
           if constexpr (kClose) mag += ok ? static_cast<R>(fabs(x[l])) : R(0);
           v[q * E + l] = ok ? x[l] : -num<D>::inf();
         }
@@ -127,7 +131,7 @@ prox_select_kernel(const D* __restrict__ in, D* __restrict__ out, int64_t m64, i
       for (int c = 0; c < C; ++c) {
         const int i = c * BT + tid;
         const D x = col[i < m ? i : 0];
-        finite = finite && fabs(x) < num<D>::inf();
+        finite = finite && x < num<D>::inf();
         if constexpr (kClose) mag += i < m ? static_cast<R>(fabs(x)) : R(0);
         v[c] = i < m ? x : -num<D>::inf();
       }
@@ -191,6 +195,8 @@ prox_select_kernel(const D* __restrict__ in, D* __restrict__ out, int64_t m64, i
             c = last < c ? last : c;
           }
         }
+        // (fewer than k + 1 parts hold an unmasked class: all of those)
+        if (c < -num<D>::max_finite()) c = -num<D>::max_finite();
         if (!(top < num<D>::inf())) c = num<D>::quiet_nan();
         cut = c;
         if constexpr (BT > 64) {
@@ -263,7 +269,7 @@ prox_select_kernel(const D* __restrict__ in, D* __restrict__ out, int64_t m64, i
           if (rec.state == SEL_DONE && rec.branch == SDCA_BRANCH_KNAPSACK) {
             const R stray = num<R>::eps() * mag / static_cast<R>(rec.n_mid);
             const int u = rec.n_hi, e = rec.n_hi + rec.n_mid;
-            const R low = static_cast<R>(e < cnt ? list[e] : cut);
+            const R low = static_cast<R>(e < cnt ? list[e] : list_rest(cut));
             // (none free: the fixing keeps its t)
             if (e == u || (u > 0 && static_cast<R>(list[u - 1]) - rec.t - rec.hi < stray) ||
                 rec.t + rec.hi - static_cast<R>(list[u]) < stray ||
@@ -406,8 +412,9 @@ prox_select_kernel(const D* __restrict__ in, D* __restrict__ out, int64_t m64, i
         else
           lt = K * (static_cast<R>(s_u) + (K - num_u) * t_fix) < rhs * (num_u + pp.rho * K * K) - eps;
         const R sum_k = static_cast<R>(ps[k]);
-        const bool constant = static_cast<R>(list[k - 1]) - sum_k / (K + pp.rho * K * K) >=
-                              static_cast<R>(list[k]) - R(16) * num<R>::eps();
+        const bool constant =
+            static_cast<R>(list[k - 1]) - sum_k / (K + pp.rho * K * K) >=
+            static_cast<R>(k < cnt ? list[k] : list_rest(cut)) - R(16) * num<R>::eps();
         rec.state = (lt && !constant) ? SEL_SLOW : SEL_DONE;
         rec.t = t;
         rec.hi = hi;
@@ -452,8 +459,10 @@ prox_select_kernel(const D* __restrict__ in, D* __restrict__ out, int64_t m64, i
           select_sync<BT>();
         }
       }
+      // (without the masked classes at the end, unless a value is not finite)
+      const int kept = cut == cut ? prefix_end<R>(whole, 0, m, -num<R>::inf()) : m;
       if (lead)
-        thresholds_sorted<D, R, true>(whole, m, pp.op, pp.lo, pp.hi, pp.rhs, pp.rho, k, rec.t, lo,
+        thresholds_sorted<D, R, true>(whole, kept, pp.op, pp.lo, pp.hi, pp.rhs, pp.rho, k, rec.t, lo,
                                       rec.hi, rec.branch, rec.n_hi, rec.n_mid);
       if constexpr (BT > 64) {
         if (threadIdx.x == 0) rec_lds = rec;

@@ -135,6 +135,14 @@ struct SelectRecord {
   int state, branch, n_hi, n_mid;
 };
 
+// A bound of the values past a list of every value at or above the cut: the
+// cut, or -inf where that is the type's lowest value (masked classes alone
+// are left then).
+template <class D>
+__device__ inline D list_rest(D cut) {
+  return cut > -num<D>::max_finite() ? cut : -num<D>::inf();
+}
+
 // The partition of the knapsack sum_i clamp(a_i - t, 0, hi) = rhs on the
 // sorted list (every value above t is in it): rank r is above t where
 // f(a_r) < rhs and at hi where f(a_r - hi) <= rhs, one rank per lane, f from
@@ -191,7 +199,7 @@ __device__ inline void list_knapsack(const D* list, const double* ps, int cnt, i
     const double top = (u > 0 ? static_cast<double>(list[u - 1]) : static_cast<double>(list[0])) - hi;
     double low = top;
     if (u < cnt) low = static_cast<double>(list[u]);
-    else if (u < m) low = static_cast<double>(cut);
+    else if (u < m && list_rest(cut) > -num<D>::inf()) low = static_cast<double>(cut);
     t_out = static_cast<R>(0.5 * (low + top));
   }
   u_out = u;
@@ -203,7 +211,7 @@ __device__ inline void list_knapsack(const D* list, const double* ps, int cnt, i
 // each |U| = u the candidate ends e of M = ranks [u, e) are tried by the
 // lanes, the smallest accepted e of the smallest u wins, as in the
 // reference's order.  The list holds the column's cnt largest values, the
-// others are at most `cut`.  Where a search for some u may continue past
+// others are at most list_rest(cut).  Where a search for some u may continue past
 // the list (no end accepted, and t not certainly above every M that would;
 // the bound of cone_biased_regs) the result is SEL_WIDER.
 template <class D, class R>
@@ -212,6 +220,7 @@ __device__ inline SelectRecord<R> list_cone(const D* list, const double* ps, int
   const int lane = static_cast<int>(threadIdx.x) & 63;
   const R eps = R(16) * num<R>::eps();
   const R K = static_cast<R>(k);
+  const R rest = static_cast<R>(list_rest(cut));
   SelectRecord<R> rec;
   rec.state = SEL_DONE;
   rec.branch = SDCA_BRANCH_SCAN;
@@ -235,7 +244,7 @@ __device__ inline SelectRecord<R> list_cone(const D* list, const double* ps, int
       const R min_m = ei > u ? static_cast<R>(list[ei - 1]) : num<R>::inf();
       const R tt = hi + t;
       const bool pass = in && max_m - eps <= tt && tt <= min_u + eps && t <= min_m + eps;
-      const R next = ei < cnt ? static_cast<R>(list[ei]) : static_cast<R>(cut);
+      const R next = ei < cnt ? static_cast<R>(list[ei]) : rest;
       const bool take = pass && (ei == m || next - eps <= t);
       const unsigned long long taken = __ballot(take);
       if (taken) {
@@ -250,7 +259,8 @@ __device__ inline SelectRecord<R> list_cone(const D* list, const double* ps, int
       // min(M) (the bound above, next the largest value still to come), the
       // search for this u is over.
       const R tol = R(2) * eps + R(8) * num<R>::eps() * dmax(fabs(t), fabs(next));
-      const bool ends = den * (t - next) > tol * (den + static_cast<R>(m - ei) * nu);
+      const bool ends = !(next > -num<R>::inf()) ||
+                        den * (t - next) > tol * (den + static_cast<R>(m - ei) * nu);
       if (e0 + 64 > cnt) {
         if (cnt < m && __ballot(in && e == cnt && (pass || !ends))) {
           rec.state = SEL_WIDER;
@@ -285,11 +295,13 @@ __device__ inline SelectRecord<R> list_record(const D* list, const double* ps, i
   rec.t = rec.hi = R(0);
   rec.branch = SDCA_BRANCH_ZERO;
   rec.n_hi = rec.n_mid = 0;
+  if (cnt < k) return rec;  // masked classes among the k largest: no sum above 0
   const R sum_k = static_cast<R>(ps[k]);
   if (sum_k <= eps16) return rec;
   const R hi_c = sum_k / (K + rho * K * K);
   const R t_c = static_cast<R>(list[k - 1]) - hi_c;
-  const bool constant = k == m || t_c >= static_cast<R>(list[k < cnt ? k : k - 1]) - eps16;
+  const bool constant =
+      k == m || t_c >= static_cast<R>(k < cnt ? list[k] : list_rest(cut)) - eps16;
   const R eps = num<R>::eps() * dmax(R(1), fabs(rhs));
   if (constant && (cone || !(K * hi_c > rhs + eps))) {
     rec.t = t_c;

@@ -1,5 +1,5 @@
 """Columns of the top-k operators whose masked classes are set to a very low
-value.  A masked class ends at 0 and takes no part in the others' thresholds,
+value or to -inf.  A masked class ends at 0 and takes no part in the others' thresholds,
 so the outputs are those of the column without it, which the CPU oracle
 computes in long double.  Sizes on every path: the register kernel and its
 deferred columns, the selection by wave and by workgroup, and its fallback to
@@ -61,3 +61,34 @@ def test_masked_low(cuda, oracle, op, kw, m, k, dtype):
     """Finite masks, down to the type's lowest value."""
     for mask in (-1e9, -1e30, -np.finfo(dtype).max):
         check_masked(oracle, cuda, op, kw, m, k, dtype, dtype(mask))
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("m,k", [(40, 20), (300, 20), (513, 3), (700, 3), (1024, 20), (1025, 8),
+                                 (2048, 3), (2049, 5), (3000, 8), (10000, 20), (16384, 10)])
+@pytest.mark.parametrize("op,kw", OPS)
+def test_masked_inf(cuda, oracle, op, kw, m, k, dtype):
+    """-inf on the selection's columns: left out like padding."""
+    check_masked(oracle, cuda, op, kw, m, k, dtype, -np.inf)
+
+
+@pytest.mark.parametrize("m,k", [(1500, 8), (2500, 5), (2500, 55)])
+def test_masked_inf_among_ties(cuda, oracle, m, k):
+    """More equal values than the selection's list holds (k < 56: its route) beside masked
+    classes: the sorted column without them."""
+    import torch
+    import libsdca_amd as sd
+    x = np.full((2, m), 0.5, np.float32)
+    x[0, 400:] = -np.inf
+    x[1, ::2] = -np.inf
+    for op, kw in OPS:
+        got = sd.prox(op, torch.from_numpy(x).to(cuda), k=k, **kw).cpu().numpy()
+        for j in range(2):
+            keep = x[j] > 0
+            n = int(keep.sum())
+            from oracle import binding
+            want = x[j, keep].astype(np.float64)[None, :].copy()
+            oracle.prox(op, want, result=2, params=binding.make_params(k=k, **kw))
+            assert (got[j, ~keep] == 0).all()
+            # one ulp of 0.5 in the threshold moves every entry together
+            assert np.abs(got[j, keep] - want[0]).max() <= 4 * np.finfo(np.float32).eps, f"{op} n={n}"

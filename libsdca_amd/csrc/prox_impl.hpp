@@ -285,18 +285,21 @@ __device__ inline KnapState<R> knapsack_eq_regs(const D (&v)[C], int m, int nval
 // sum over the values still free, not updated from the previous one: that
 // keeps the large fixed values out of the final sum, as the reference's
 // sum over M does.
+//
+// floor: the values at or below it are fixed at lo from the start (-inf:
+// none); the caller knows that they end there, and `total` leaves them out.
 template <int G, int C, class D, class R>
 __device__ inline R knapsack_biased_regs(const D (&v)[C], int m, R total, R lo, R hi, R rhs,
-                                         R rho_inv) {
+                                         R rho_inv, R floor = -num<R>::inf(), int n_floor = 0) {
   const R eps = num<R>::eps() * dmax(R(1), fabs(rhs));
   const R qnan = num<R>::quiet_nan();
-  int n_l = 0, n_u = 0;
+  int n_l = n_floor, n_u = 0;
   R s_free = total;
   R w[C];
 #pragma unroll
   for (int c = 0; c < C; ++c) {
     const R x = static_cast<R>(v[c]);
-    w[c] = (x > -num<R>::inf()) ? x : qnan;
+    w[c] = (x > floor) ? x : qnan;
   }
   R t = 0;
   for (int iter = 0; iter <= m; ++iter) {
@@ -336,6 +339,46 @@ __device__ inline R knapsack_biased_regs(const D (&v)[C], int m, R total, R lo, 
   return t;
 }
 
+// knapsack_le_biased on a workgroup's column with masked classes: values at
+// -inf, or so low that the column's sum is -inf, from which the fixing cannot
+// start.  Each fixing here starts without the values that certainly end at
+// lo: a value at or below lo + (a lower bound of t) does.
+template <int G, int C, class D, class R, class S>
+__device__ inline ColThr<R> knapsack_le_biased_masked(const D (&v)[C], int m, int nvalid,
+                                                      const ProxParamsT<R>& pp) {
+  const R lo = pp.lo, hi = pp.hi, rhs = pp.rhs, rho = pp.rho;
+  const R eps = num<R>::eps() * dmax(R(1), fabs(rhs));
+  auto above = [&](R cut, S& sum, int& count) {
+    sum = 0;
+    count = 0;
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      const R x = static_cast<R>(v[c]);
+      sum += x > cut ? x : R(0);
+      count += x > cut ? 1 : 0;
+    }
+    group_sums<G>(sum, count);
+  };
+  S sum;
+  int count;
+  // Without the sum constraint t = rho sum x >= rho m lo.
+  const R bound = lo + rho * (static_cast<R>(m) * lo);
+  const R floor = bound - fabs(bound) * (R(16) * num<R>::eps());
+  above(floor, sum, count);
+  const R t = knapsack_biased_regs<G, C, D, R>(v, m, static_cast<R>(sum), lo, hi, rhs, R(1) / rho,
+                                               floor, m - count);
+  if (t <= rho * rhs + eps) return tag_thr(make_thr<R>(t, lo, hi), SDCA_BRANCH_SCAN);
+  // With it x sums to less, so its t is above this one.
+  const R cut = lo + t;
+  above(cut, sum, count);
+  D w[C];
+#pragma unroll
+  for (int c = 0; c < C; ++c) w[c] = static_cast<R>(v[c]) > cut ? v[c] : -num<D>::inf();
+  const KnapState<R> st = knapsack_eq_regs<G, C, D, R, false, S>(
+      w, count, nvalid, static_cast<R>(sum), lo, hi, rhs - lo * static_cast<R>(m - count));
+  return tag_thr(make_thr<R>(st.t_acc, lo, hi), SDCA_BRANCH_KNAPSACK, st.n_u, st.n_f);
+}
+
 // ---------------------------------------------------------------------------
 // Knapsack family: knapsack_eq (knapsack_eq.h:25-109) and knapsack_le
 // (knapsack_le.h:17-44).  MAX_START: the start from the bound max - rhs below
@@ -368,6 +411,22 @@ __device__ inline ColThr<R> knap_family(const D (&v)[C], int m, int nvalid,
   R total = 0;
   // Columns held by a workgroup of 512 threads or more sum in double.
   typedef typename std::conditional<(G >= 512), double, R>::type S;
+  if constexpr (G >= 512) {
+    if (biased) {
+      S sum = 0;
+      int masked = 0;
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        const R x = static_cast<R>(v[c]);
+        sum += (c < nvalid && x != -num<R>::inf()) ? x : R(0);
+        masked += (c < nvalid && x == -num<R>::inf()) ? 1 : 0;
+      }
+      group_sums<G>(sum, masked);
+      const R low = static_cast<R>(sum);
+      if (low == -num<R>::inf() || (masked > 0 && low < num<R>::inf()))
+        return knapsack_le_biased_masked<G, C, D, R, S>(v, m, nvalid, pp);
+    }
+  }
   // With lo = 0 and hi >= rhs the largest entry alone can take the whole
   // sum, so t >= max - rhs: the entries below that bound end at 0 and are
   // left out (as padding) from the start.  Kiwiel's start at the mean halves

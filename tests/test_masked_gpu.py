@@ -92,3 +92,40 @@ def test_masked_inf_among_ties(cuda, oracle, m, k):
             assert (got[j, ~keep] == 0).all()
             # one ulp of 0.5 in the threshold moves every entry together
             assert np.abs(got[j, keep] - want[0]).max() <= 4 * np.finfo(np.float32).eps, f"{op} n={n}"
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("m", [2049, 3000, 16384])
+@pytest.mark.parametrize("lo", [0.0, -1e-3])
+def test_masked_knapsack_le_biased(cuda, m, lo, dtype):
+    """knapsack_le_biased on a workgroup's columns whose sum is -inf (two
+    classes or more at the type's lowest value, one at -inf):
+    x = clamp(a - t, lo, 1) with t = rho sum x where that sum is at most 1,
+    else sum x = 1."""
+    import torch
+    import libsdca_amd as sd
+    rho = 0.5
+    u = float(np.finfo(dtype).eps)
+    for mask in (-np.inf, -np.finfo(dtype).max):
+        # 3 and 4 classes at 0.3: inactive for lo = 0; 16 with a label: active
+        cols = []
+        for kept, scale in ((3, 0.1), (4, 0.3), (16, 1.0), (m // 2, 1.0), (m - 2, 1.0)):
+            rng = np.random.default_rng(m + kept)
+            x = np.full(m, mask)
+            x[rng.permutation(m)[:kept]] = rng.standard_normal(kept) * scale + 0.1
+            cols.append(x)
+        x = np.stack(cols).astype(dtype)
+        got, thr = sd.prox("knapsack_le_biased", torch.from_numpy(x).to(cuda), lo=lo, rho=rho,
+                           thresholds=True)
+        got, thr = got.cpu().numpy().astype(np.float64), thr.cpu().numpy()
+        for j in range(len(x)):
+            keep = x[j] > -1e30
+            t, s = thr[j, 0], got[j].sum()
+            assert (got[j, ~keep] == float(dtype(lo))).all(), (j, mask)
+            # the outputs' own rounding in the sum: m u of values up to 4
+            tol = 8 * m * u
+            assert np.abs(got[j, keep] - np.clip(x[j, keep] - t, lo, 1.0)).max() <= 8 * u
+            if s <= 1.0 - tol:
+                assert abs(t - rho * s) <= tol, (j, mask, t, s)
+            else:
+                assert abs(s - 1.0) <= tol and t >= rho * 1.0 - tol, (j, mask, t, s)

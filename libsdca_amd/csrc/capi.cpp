@@ -446,12 +446,14 @@ int prox_entry(int op_in, int data_in, int result_in, int64_t m, int64_t n, cons
     SDCA_HIP_TRY(launch_ent_biased(a), "topk_entropy_biased kernel (wave per column)");
   } else if (topk_like &&
              (!topk_in_registers(op, data, m, p.k) ||
+              (p.k > 8 && n > kTopkRegMaxColumns) ||
               (p.k > 8 && !fixed_list &&
                !list_available(stream, static_cast<size_t>(n + 2) * sizeof(int))))) {
     // Columns beyond the register kernel: by selection, or for the largest
-    // k one workgroup per sorted column.  With k > 8 also where the
-    // register kernel's list of deferred columns would have to be allocated
-    // under capture: these calls need no scratch.
+    // k one workgroup per sorted column.  With k > 8 also for more columns
+    // than one launch of the register kernel takes, and where its list of
+    // deferred columns would have to be allocated under capture: these calls
+    // need no scratch.
     if (select_supported(a))
       SDCA_HIP_TRY(launch_select(a, true), "prox kernel (selection)");
     else

@@ -25,7 +25,6 @@ hipError_t launch_one(const ProxLaunch& a) {
   pp.rhs_k = (a.k > 0) ? pp.rhs / static_cast<R>(a.k) : R(0);
   pp.op = a.op;
   pp.p = static_cast<int>(a.p);
-  const int64_t blocks = (a.n + B - 1) / B;
   // B*m tile, G*C - m words of slack for branch-free slot reads (slot c of
   // the last column's lane g is word (B - 1) m + g + G c <= B m + G C - m - 1),
   // BT dummy words.  Slack of G*C - m words rather than G*C keeps the LDS
@@ -63,20 +62,26 @@ hipError_t launch_one(const ProxLaunch& a) {
   // m == G * C (the configuration's exact size) gets the variant without
   // per-slot validity tests (for one-wave workgroups: the wide
   // configurations are for rare sizes and keep one variant).
+  auto kernel = &prox_columns_kernel<FAM, KM, D, R, G, C, BT, false>;
   if constexpr (BT == 64) {
-    if (full) {
-      hipLaunchKernelGGL((prox_columns_kernel<FAM, KM, D, R, G, C, BT, true>),
-                         dim3(static_cast<unsigned>(blocks)), dim3(BT), shmem, a.stream,
-                         static_cast<const D*>(a.in), static_cast<D*>(a.out), a.m, a.n, pp,
-                         a.col_p, a.thr, a.slow, a.sets);
-      return hipGetLastError();
-    }
+    if (full) kernel = &prox_columns_kernel<FAM, KM, D, R, G, C, BT, true>;
   }
-  hipLaunchKernelGGL((prox_columns_kernel<FAM, KM, D, R, G, C, BT, false>),
-                     dim3(static_cast<unsigned>(blocks)), dim3(BT), shmem, a.stream,
-                     static_cast<const D*>(a.in), static_cast<D*>(a.out), a.m, a.n, pp,
-                     a.col_p, a.thr, a.slow, a.sets);
-  return hipGetLastError();
+  // One launch, or as many as the columns need (a list of deferred columns
+  // holds column ids of the one launch: refused beyond it).
+  constexpr int64_t kRecords = FAM == FAM_TWO ? 2 : 1;  // threshold records per column
+  const int64_t most = max_blocks(BT) * B;
+  if (a.slow && a.n > most) return hipErrorInvalidConfiguration;
+  for (int64_t j = 0; j < a.n; j += most) {
+    const int64_t n = a.n - j < most ? a.n - j : most;
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>((n + B - 1) / B)), dim3(BT), shmem,
+                       a.stream, static_cast<const D*>(a.in) + j * a.m,
+                       static_cast<D*>(a.out) + j * a.m, a.m, n, pp,
+                       a.col_p ? a.col_p + j : nullptr, a.thr ? a.thr + kRecords * j : nullptr,
+                       a.slow, a.sets ? a.sets + kRecords * j : nullptr);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 // Columns above kRegMaxM rows: one workgroup per column (kWideThreads

@@ -42,6 +42,14 @@ constexpr int64_t kMaxColumnBytes = 128 * 1024;
 inline int64_t max_rows(int data) {
   return kMaxColumnBytes / (data == SDCA_F32 ? 4 : 8);
 }
+// A launch holds fewer than 2^32 threads (HIP refuses that many, and beyond
+// it starts the count modulo 2^32): the most workgroups of `threads` threads
+// in one launch.
+inline int64_t max_blocks(int threads) { return ((int64_t(1) << 32) - 1) / threads; }
+// Columns from which on the top-k operators with k > 8 leave the register
+// kernel (up to 16 lanes per column, one launch, for the list's column ids)
+// for the selection, whose workgroups take columns in turn.
+constexpr int64_t kTopkRegMaxColumns = (int64_t(1) << 28) - 1;
 // Whether the register kernel takes a top-k operator's columns: its sorted
 // lists hold k <= 8 of a column (k <= 15 with the longest list, which pays
 // where several columns share a wave: 40e6 fp32 entries of m = 100, k = 10,

@@ -547,7 +547,7 @@ hipError_t select_one(const ProxLaunch& a, bool all_columns) {
   // little to launch.
   const int64_t groups = (a.n + NG - 1) / NG;
   const int64_t work = a.n * a.m / 16384;
-  const int64_t cap = all_columns ? (int64_t(1) << 30)
+  const int64_t cap = all_columns ? max_blocks(BT > 64 ? BT : 64 * NG)
                                   : std::min<int64_t>(1024, std::max<int64_t>(256, work));
   const int64_t grid = std::max<int64_t>(1, std::min(groups, cap));
   hipLaunchKernelGGL((prox_select_kernel<D, R, BT, C>), dim3(static_cast<unsigned>(grid)),

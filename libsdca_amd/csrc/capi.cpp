@@ -107,19 +107,14 @@ int workspace(hipStream_t stream, int slot, size_t bytes, void** out, Workspace*
   return SDCA_OK;
 }
 
-// Whether the deferred-column list (slot 0) of `bytes` can be had: not under
-// graph capture beyond what the stream already has.
-bool list_available(hipStream_t stream, size_t bytes) {
+// Whether the stream is being captured (or cannot be asked).
+bool capturing(hipStream_t stream) {
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(stream, &cs) != hipSuccess) {
     (void)hipGetLastError();
     return true;
   }
-  if (cs == hipStreamCaptureStatusNone) return true;
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return true;
-  std::lock_guard<std::mutex> lock(g_ws_mutex);
-  return g_ws[std::make_tuple(dev, stream, std::this_thread::get_id())].cap[0] >= bytes;
+  return cs != hipStreamCaptureStatusNone;
 }
 
 // The library GEMM's workspace (slot 5) for an fp32 score GEMM of n m d:
@@ -446,14 +441,12 @@ int prox_entry(int op_in, int data_in, int result_in, int64_t m, int64_t n, cons
     SDCA_HIP_TRY(launch_ent_biased(a), "topk_entropy_biased kernel (wave per column)");
   } else if (topk_like &&
              (!topk_in_registers(op, data, m, p.k) ||
-              (p.k > 8 && n > kTopkRegMaxColumns) ||
-              (p.k > 8 && !fixed_list &&
-               !list_available(stream, static_cast<size_t>(n + 2) * sizeof(int))))) {
+              (p.k > 8 && (n > kTopkRegMaxColumns || (!fixed_list && capturing(stream)))))) {
     // Columns beyond the register kernel: by selection, or for the largest
     // k one workgroup per sorted column.  With k > 8 also for more columns
-    // than one launch of the register kernel takes, and where its list of
-    // deferred columns would have to be allocated under capture: these calls
-    // need no scratch.
+    // than one launch of the register kernel takes, and under capture: these
+    // calls need no scratch, so a graph of them holds no pointer to the list
+    // of deferred columns, which a later, larger call on the stream frees.
     if (select_supported(a))
       SDCA_HIP_TRY(launch_select(a, true), "prox kernel (selection)");
     else

@@ -361,6 +361,53 @@ __device__ inline double xor_lane(double v) {
                               (static_cast<long long>(static_cast<unsigned>(lo))));
 }
 
+// A double sum with the rounding of its additions beside it (Neumaier): what
+// double sums are carried in where R alone would round on every addition, as
+// double carries float sums.  (A sum that is not finite has no compensation.)
+struct SumPair {
+  double s, c;
+  SumPair() = default;
+  __device__ SumPair(double x) : s(x), c(0.0) {}
+  __device__ SumPair& operator+=(double x) {
+    const double t = s + x;
+    c += (fabs(s) >= fabs(x)) ? (s - t) + x : (x - t) + s;
+    s = t;
+    return *this;
+  }
+  // (commutative to the bit: both lanes of an exchange end with the same)
+  __device__ SumPair& operator+=(const SumPair& b) {
+    const double t = s + b.s;
+    c = (c + b.c) + ((fabs(s) >= fabs(b.s)) ? (s - t) + b.s : (b.s - t) + s);
+    s = t;
+    return *this;
+  }
+  __device__ explicit operator double() const {
+    return fabs(s) < num<double>::inf() ? s + c : s;
+  }
+};
+__device__ inline SumPair operator+(SumPair a, const SumPair& b) { return a += b; }
+// s += x where b: a select for the plain sums, a branch for the pairs (their
+// addition is nine instructions, and a wave often has no value to add).
+template <class S, class R>
+__device__ inline void add_if(S& s, bool b, R x) {
+  s += b ? x : R(0);
+}
+__device__ inline void add_if(SumPair& s, bool b, double x) {
+  if (b) s += x;
+}
+template <int OFF, bool VALU = false>
+__device__ inline SumPair xor_lane(const SumPair& v) {
+  SumPair r;
+  r.s = xor_lane<OFF, VALU>(v.s);
+  r.c = xor_lane<OFF, VALU>(v.c);
+  return r;
+}
+// The type that sums of R are carried in where one rounding at the end is
+// wanted.
+template <class R> struct WideSum;
+template <> struct WideSum<float> { typedef double type; };
+template <> struct WideSum<double> { typedef SumPair type; };
+
 // ---------------------------------------------------------------------------
 // Reductions over a group of G adjacent lanes of a wave (G a power of two,
 // groups aligned to G).  Every lane of the group receives the result.
@@ -480,6 +527,12 @@ __device__ inline T wave_total(T x) {
   return lane63(x);
 }
 
+__device__ inline SumPair wave_total(SumPair x) {
+  // (often no lane has a term: the six exchanges are a long chain)
+  if (!__ballot(x.s != 0.0 || x.c != 0.0)) return SumPair(0.0);
+  return lanes_sum<64, true>(x);
+}
+
 template <int G, class T>
 __device__ inline T group_sum(T x) {
   if constexpr (G > 64) {
@@ -492,8 +545,9 @@ __device__ inline T group_sum(T x) {
 // would, the workgroup-wide ones through one pair of barriers for all of
 // them (the same wave-order sums, so the same bits as separate calls).
 template <class T>
+constexpr int kSlotWords = static_cast<int>((sizeof(T) + 7) / 8);
+template <class T>
 __device__ inline void slot_put(unsigned long long& slot, T x) {
-  static_assert(sizeof(T) <= sizeof(unsigned long long), "8-byte slots");
   __builtin_memcpy(&slot, &x, sizeof(T));
 }
 template <class T>
@@ -511,7 +565,7 @@ __device__ inline T slot_sum(const unsigned long long (*slots)[8], int i) {
 }
 template <int G, class... T>
 __device__ inline void group_sums(T&... x) {
-  static_assert(sizeof...(T) <= 8, "at most 8 values per exchange");
+  static_assert((kSlotWords<T> + ... + 0) <= 8, "at most 8 words per exchange");
   if constexpr (G > 64) {
     __shared__ unsigned long long slots[kMaxGroupWaves][8];
     ((x = wave_total(x)), ...);
@@ -519,11 +573,11 @@ __device__ inline void group_sums(T&... x) {
     if ((threadIdx.x & 63) == 0) {
       const int w = static_cast<int>(threadIdx.x) >> 6;
       int i = 0;
-      ((slot_put(slots[w][i++], x)), ...);
+      ((slot_put(slots[w][i], x), i += kSlotWords<T>), ...);
     }
     __syncthreads();
     int i = 0;
-    ((x = slot_sum<G, T>(slots, i++)), ...);
+    ((x = slot_sum<G, T>(slots, i), i += kSlotWords<T>), ...);
   } else {
     ((x = group_sum<G>(x)), ...);
   }

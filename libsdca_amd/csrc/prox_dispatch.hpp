@@ -88,8 +88,10 @@ hipError_t launch_one(const ProxLaunch& a) {
 // threads, kMaxWideThreads for the largest fp32 columns), C slots per
 // thread; the column (at most kMaxColumnBytes) is staged in LDS and the
 // group reductions combine the waves through LDS.  (The knapsack, 40e6 fp32
-// entries: m = 3000 359 us, 8000 249, 16000 324, 30000 417, against 2286,
-// 2495, 4893 and 11745 with the column sorted in LDS.)
+// entries: m = 3000 361 us, 8000 250, 16000 259, 30000 395, against 2286,
+// 2495, 4893 and 11745 with the column sorted in LDS; 20e6 fp64 entries, with
+// compensated sums: m = 3000 220, 8000 192, 16000 167, against 1556, 2349 and
+// 4693.)
 template <int FAM, int KM, class D, class R>
 hipError_t launch_wide(const ProxLaunch& a) {
   constexpr int G = kWideThreads, G2 = kMaxWideThreads;
@@ -106,6 +108,11 @@ hipError_t launch_wide(const ProxLaunch& a) {
 template <int FAM, int KM, class D, class R>
 hipError_t launch_by_m(const ProxLaunch& a) {
   // The top-k family's columns above 1024 rows go by selection.
+  if constexpr (FAM == FAM_KNAP) {
+    // (KM = 1: the biased knapsack's own kernel)
+    if (a.m > kRegMaxM && a.op == OP_KNAPSACK_LE_BIASED && static_cast<R>(a.rho) != R(0))
+      return launch_wide<FAM, 1, D, R>(a);
+  }
   if constexpr (FAM != FAM_TOPK) {
     if (a.m > kRegMaxM) return launch_wide<FAM, KM, D, R>(a);
   }

@@ -88,10 +88,11 @@ __device__ inline ColThr<R> slow_thr() {
   return r;
 }
 
-// Sum of the valid slots (padding, and excluded slots, hold -inf).
-template <int G, int C, class D, class R>
-__device__ inline R total_sum(const D (&v)[C], int nvalid) {
-  R s = 0;
+// Sum of the valid slots (padding, and excluded slots, hold -inf), carried
+// in S.
+template <int G, int C, class D, class R, class S = R>
+__device__ inline S total_sum(const D (&v)[C], int nvalid) {
+  S s = 0;
 #pragma unroll
   for (int c = 0; c < C; ++c) {
     const R x = static_cast<R>(v[c]);
@@ -120,7 +121,8 @@ struct KnapState {
 
 // The fixing may start with the n_u0 values above hi_cut0 (sum sum_u0)
 // already at the upper bound, when those are known to end there; the
-// iteration is then Kiwiel's on the remaining problem.
+// iteration is then Kiwiel's on the remaining problem.  The values at or
+// below lo_cut0 are left out like padding (m does not count them).
 //
 // Each lane keeps a working copy w of its slots in which every fixed value
 // (and padding) is NaN: both candidate tests (w <= lo + t, w > hi + t) are
@@ -133,12 +135,14 @@ struct KnapState {
 // their stores go to the lane's dummy word) instead of C more registers.
 // The caller must not need the LDS copy of the column afterwards.
 //
-// S: the type of the sum over the final free set.
+// S: the type every pass's sums are carried in (R, or WideSum<R>: rounded to
+// R once).
 template <int G, int C, class D, class R, bool WL = false, class S = R>
 __device__ inline KnapState<R> knapsack_eq_regs(const D (&v)[C], int m, int nvalid, R total,
                                                 R lo, R hi, R rhs, R hi_cut0 = num<R>::inf(),
                                                 int n_u0 = 0, R sum_u0 = 0, D* wl = nullptr,
-                                                D* wl_dummy = nullptr) {
+                                                D* wl_dummy = nullptr,
+                                                R lo_cut0 = -num<R>::inf()) {
   const R eps = num<R>::eps() * dmax(R(1), fabs(rhs));
   const R qnan = num<R>::quiet_nan();
   R w[WL ? 1 : C];
@@ -181,7 +185,7 @@ __device__ inline KnapState<R> knapsack_eq_regs(const D (&v)[C], int m, int nval
 #pragma unroll UW
   for (int c = 0; c < C; ++c) {
     const R x = static_cast<R>(v[c]);
-    put(c, (x > -num<R>::inf() && !(x > hi_cut0)) ? x : qnan);
+    put(c, (x > lo_cut0 && !(x > hi_cut0)) ? x : qnan);
   }
   for (int iter = 0; iter <= m; ++iter) {
     const R c_lo = lo + t, c_hi = hi + t;
@@ -192,8 +196,8 @@ __device__ inline KnapState<R> knapsack_eq_regs(const D (&v)[C], int m, int nval
       const R wc = get(c);
       const bool lo_c = wc <= c_lo;
       const bool hi_c = wc > c_hi;
-      sum_lo += lo_c ? wc : R(0);
-      sum_hi += hi_c ? wc : R(0);
+      add_if(sum_lo, lo_c, wc);
+      add_if(sum_hi, hi_c, wc);
       n_lh += (lo_c ? 1 : 0) + (hi_c ? 0x10000 : 0);
     }
     group_sums<G>(sum_lo, sum_hi, n_lh);
@@ -253,7 +257,7 @@ __device__ inline KnapState<R> knapsack_eq_regs(const D (&v)[C], int m, int nval
 #pragma unroll UW
     for (int c = 0; c < C; ++c) {
       const R wc = get(c);
-      s_f += static_cast<S>((wc > st.c_lo && !(wc > st.c_hi)) ? wc : R(0));
+      add_if(s_f, wc > st.c_lo && !(wc > st.c_hi), wc);
     }
     s_f = group_sum<G>(s_f);
     const int n_l = m - st.n_u - n_f;
@@ -288,7 +292,8 @@ __device__ inline KnapState<R> knapsack_eq_regs(const D (&v)[C], int m, int nval
 //
 // floor: the values at or below it are fixed at lo from the start (-inf:
 // none); the caller knows that they end there, and `total` leaves them out.
-template <int G, int C, class D, class R>
+// S as in knapsack_eq_regs.
+template <int G, int C, class D, class R, class S = R>
 __device__ inline R knapsack_biased_regs(const D (&v)[C], int m, R total, R lo, R hi, R rhs,
                                          R rho_inv, R floor = -num<R>::inf(), int n_floor = 0) {
   const R eps = num<R>::eps() * dmax(R(1), fabs(rhs));
@@ -308,136 +313,49 @@ __device__ inline R knapsack_biased_regs(const D (&v)[C], int m, R total, R lo, 
         (rho_inv + static_cast<R>(n_m));
     if (n_m == 0) break;
     const R c_lo = lo + t, c_hi = hi + t;
-    R s_lo = 0, s_hi = 0;
+    S sum_lo = 0, sum_hi = 0;
     int n_lh = 0;
 #pragma unroll
     for (int c = 0; c < C; ++c) {
       const bool lo_c = w[c] <= c_lo;
       const bool hi_c = w[c] > c_hi;
-      s_lo += lo_c ? w[c] : R(0);
-      s_hi += hi_c ? w[c] : R(0);
+      add_if(sum_lo, lo_c, w[c]);
+      add_if(sum_hi, hi_c, w[c]);
       n_lh += (lo_c ? 1 : 0) + (hi_c ? 0x10000 : 0);
     }
-    group_sums<G>(s_lo, s_hi, n_lh);
+    group_sums<G>(sum_lo, sum_hi, n_lh);
+    const R s_lo = static_cast<R>(sum_lo), s_hi = static_cast<R>(sum_hi);
     const int n_lo = n_lh & 0xffff, n_hi = static_cast<int>(static_cast<unsigned>(n_lh) >> 16);
     const R infeas = s_hi + s_lo - (static_cast<R>(n_hi) * hi + static_cast<R>(n_lo) * lo) -
                      static_cast<R>(n_hi + n_lo) * t;
     const bool fix_hi = n_hi > 0 && infeas > eps;
     const bool fix_lo = !fix_hi && n_lo > 0 && infeas < -eps;
     if (!fix_hi && !fix_lo) break;
-    R sf = 0;
+    S sf = 0;
 #pragma unroll
     for (int c = 0; c < C; ++c) {
       const bool fixed = fix_hi ? (w[c] > c_hi) : (w[c] <= c_lo);
       w[c] = fixed ? qnan : w[c];
-      sf += (w[c] == w[c]) ? w[c] : R(0);
+      add_if(sf, w[c] == w[c], w[c]);
     }
-    s_free = group_sum<G>(sf);
+    s_free = static_cast<R>(group_sum<G>(sf));
     if (fix_hi) n_u += n_hi;
     else n_l += n_lo;
   }
   return t;
 }
 
-// knapsack_le_biased on a workgroup's column with masked classes: values at
-// -inf, or so low that the column's sum is -inf, from which the fixing cannot
-// start.  Each fixing here starts without the values that certainly end at
-// lo: a value at or below lo + (a lower bound of t) does.
-template <int G, int C, class D, class R, class S>
-__device__ inline ColThr<R> knapsack_le_biased_masked(const D (&v)[C], int m, int nvalid,
-                                                      const ProxParamsT<R>& pp) {
-  const R lo = pp.lo, hi = pp.hi, rhs = pp.rhs, rho = pp.rho;
-  const R eps = num<R>::eps() * dmax(R(1), fabs(rhs));
-  auto above = [&](R cut, S& sum, int& count) {
-    sum = 0;
-    count = 0;
-#pragma unroll
-    for (int c = 0; c < C; ++c) {
-      const R x = static_cast<R>(v[c]);
-      sum += x > cut ? x : R(0);
-      count += x > cut ? 1 : 0;
-    }
-    group_sums<G>(sum, count);
-  };
-  S sum;
-  int count;
-  // Without the sum constraint t = rho sum x >= rho m lo.
-  const R bound = lo + rho * (static_cast<R>(m) * lo);
-  const R floor = bound - fabs(bound) * (R(16) * num<R>::eps());
-  above(floor, sum, count);
-  const R t = knapsack_biased_regs<G, C, D, R>(v, m, static_cast<R>(sum), lo, hi, rhs, R(1) / rho,
-                                               floor, m - count);
-  if (t <= rho * rhs + eps) return tag_thr(make_thr<R>(t, lo, hi), SDCA_BRANCH_SCAN);
-  // With it x sums to less, so its t is above this one.
-  const R cut = lo + t;
-  above(cut, sum, count);
-  D w[C];
-#pragma unroll
-  for (int c = 0; c < C; ++c) w[c] = static_cast<R>(v[c]) > cut ? v[c] : -num<D>::inf();
-  const KnapState<R> st = knapsack_eq_regs<G, C, D, R, false, S>(
-      w, count, nvalid, static_cast<R>(sum), lo, hi, rhs - lo * static_cast<R>(m - count));
-  return tag_thr(make_thr<R>(st.t_acc, lo, hi), SDCA_BRANCH_KNAPSACK, st.n_u, st.n_f);
-}
-
-// ---------------------------------------------------------------------------
-// Knapsack family: knapsack_eq (knapsack_eq.h:25-109) and knapsack_le
-// (knapsack_le.h:17-44).  MAX_START: the start from the bound max - rhs below
-// (the prox kernels).  The SDCA epoch goes without it: its hinge takes that
-// start at k = 1 only, and carried its exchange buffer (1 KiB of LDS), up to
-// nine registers and the spilled scalars of its branch for every other k.
-// ---------------------------------------------------------------------------
-template <int G, int C, class D, class R, bool MAX_START = true>
-__device__ inline ColThr<R> knap_family(const D (&v)[C], int m, int nvalid,
-                                        const ProxParamsT<R>& pp) {
-  const R lo = pp.lo, hi = pp.hi, rhs = pp.rhs;
-  // knapsack_le_biased with rho = 0 is knapsack_le (knapsack_le_biased.h:113-115).
-  const bool biased = pp.op == OP_KNAPSACK_LE_BIASED && pp.rho != R(0);
-  if (pp.op == OP_KNAPSACK_LE || (pp.op == OP_KNAPSACK_LE_BIASED && !biased)) {
-    const R eps = num<R>::eps() * dmax(R(1), fabs(rhs));
-    R s_mid = 0;
-    int n_hi = 0, n_mid = 0;
-#pragma unroll
-    for (int c = 0; c < C; ++c) {
-      const R x = static_cast<R>(v[c]);
-      if (x >= hi) ++n_hi;
-      else if (x > lo) { s_mid += x; ++n_mid; }
-    }
-    group_sums<G>(s_mid, n_hi, n_mid);
-    const int n_lo = m - n_hi - n_mid;
-    const R s = s_mid + hi * static_cast<R>(n_hi) + lo * static_cast<R>(n_lo);
-    if (!(s > rhs + eps)) return tag_thr(make_thr<R>(R(0), lo, hi), SDCA_BRANCH_INACTIVE, n_hi, n_mid);
-  }
-  KnapState<R> st;
-  R total = 0;
-  // Columns held by a workgroup of 512 threads or more sum in double.
-  typedef typename std::conditional<(G >= 512), double, R>::type S;
-  if constexpr (G >= 512) {
-    if (biased) {
-      S sum = 0;
-      int masked = 0;
-#pragma unroll
-      for (int c = 0; c < C; ++c) {
-        const R x = static_cast<R>(v[c]);
-        sum += (c < nvalid && x != -num<R>::inf()) ? x : R(0);
-        masked += (c < nvalid && x == -num<R>::inf()) ? 1 : 0;
-      }
-      group_sums<G>(sum, masked);
-      const R low = static_cast<R>(sum);
-      if (low == -num<R>::inf() || (masked > 0 && low < num<R>::inf()))
-        return knapsack_le_biased_masked<G, C, D, R, S>(v, m, nvalid, pp);
-    }
-  }
-  // With lo = 0 and hi >= rhs the largest entry alone can take the whole
-  // sum, so t >= max - rhs: the entries below that bound end at 0 and are
-  // left out (as padding) from the start.  Kiwiel's start at the mean halves
-  // the free set about once per pass instead; what remains above the bound
-  // of an N(0,1) column is a handful of entries (40e6 fp32 entries: m = 100
-  // 87 -> 63 us, 300 174 -> 128, 1000 103 -> 68).  Not for a workgroup's
-  // float column: there the rounding of the fixing's numerator (sums of
-  // thousands over a dozen free values) decides which values near t are free,
-  // and it takes the sorted column's steps from the mean on.
-  const bool from_max = MAX_START && sizeof(S) == sizeof(R) && lo == R(0) && hi >= rhs;
-  if (from_max) {
+// The equality's solution over the column (knapsack_eq.h:25-109).  MAX_START:
+// where lo = 0 and hi >= rhs the largest entry alone can take the whole sum,
+// so t >= max - rhs: the entries below that bound end at 0 and are left out
+// (as padding) from the start.  Kiwiel's start at the mean halves the free
+// set about once per pass instead; what remains above the bound of an N(0,1)
+// column is a handful of entries (40e6 fp32 entries: m = 100 87 -> 63 us,
+// 300 174 -> 128, 1000 103 -> 68).
+template <int G, int C, class D, class R, class S, bool MAX_START>
+__device__ inline KnapState<R> knap_equality(const D (&v)[C], int m, int nvalid, R lo, R hi,
+                                             R rhs) {
+  if (MAX_START && lo == R(0) && hi >= rhs) {
     R mx = -num<R>::inf(), sum = 0;
 #pragma unroll
     for (int c = 0; c < C; ++c) {
@@ -452,37 +370,140 @@ __device__ inline ColThr<R> knap_family(const D (&v)[C], int m, int nvalid,
     const R cut = mx - rhs - (fabs(mx) + rhs) * (R(16) * num<R>::eps());
     const bool every = !(mx < num<R>::inf());
     D w[C];
-    R s_c = 0;
+    S s_c = 0;
     int n_c = 0;
 #pragma unroll
     for (int c = 0; c < C; ++c) {
       const R x = static_cast<R>(v[c]);
       const bool in = c < nvalid && (every || x >= cut);
       w[c] = in ? v[c] : -num<D>::inf();
-      s_c += (in && x > -num<R>::inf()) ? x : R(0);
+      add_if(s_c, in && x > -num<R>::inf(), x);
       n_c += in ? 1 : 0;
     }
     group_sums<G>(s_c, n_c);
-    st = knapsack_eq_regs<G, C, D, R, false, S>(w, n_c, nvalid, s_c, lo, hi, rhs);
-  } else {
-    total = static_cast<R>(total_sum<G, C, D, S>(v, nvalid));
-    st = knapsack_eq_regs<G, C, D, R, false, S>(v, m, nvalid, total, lo, hi, rhs);
+    return knapsack_eq_regs<G, C, D, R, false, S>(w, n_c, nvalid, static_cast<R>(s_c), lo, hi, rhs);
   }
-  if (biased) {
-    // knapsack_le_biased.h:117-128: the equality solution stands if
-    // t >= rho rhs - eps; otherwise the sum constraint is inactive.
-    const R eps = num<R>::eps() * dmax(R(1), fabs(rhs));
-    if (!(st.t >= pp.rho * rhs - eps)) {
-      if (from_max) total = total_sum<G, C, D, R>(v, nvalid);
-      return tag_thr(make_thr<R>(knapsack_biased_regs<G, C, D, R>(v, m, total, lo, hi, rhs,
-                                                                  R(1) / pp.rho),
-                                 lo, hi),
-                     SDCA_BRANCH_SCAN);
+  const R total = static_cast<R>(total_sum<G, C, D, R, S>(v, nvalid));
+  return knapsack_eq_regs<G, C, D, R, false, S>(v, m, nvalid, total, lo, hi, rhs);
+}
+
+// knapsack_le_biased with rho > 0 (knapsack_le_biased.h:94-137) on a
+// workgroup's column: the equality solution if its t is at least rho rhs,
+// else the search's.
+//
+// A column with masked classes, at -inf or so low that the column's sum is
+// -inf, gives the equality no sum to start from.  It takes the search first,
+// without the values that certainly end at lo (at or below lo + a lower
+// bound of t: without the sum constraint t = rho sum x >= rho m lo); if that
+// t breaks the constraint, x sums to less and t is larger, so the equality
+// then starts without the values at or below lo + t.
+template <int G, int C, class D, class R, class S, bool MAX_START>
+__device__ inline ColThr<R> knapsack_le_biased_wide(const D (&v)[C], int m, int nvalid,
+                                                    const ProxParamsT<R>& pp) {
+  const R lo = pp.lo, hi = pp.hi, rhs = pp.rhs, rho = pp.rho;
+  const R eps = num<R>::eps() * dmax(R(1), fabs(rhs));
+  R sum = 0;      // of the values above a cut
+  int count = 0;  // and their number
+  auto above = [&](R cut) {
+    S s = 0;
+    count = 0;
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      const R x = static_cast<R>(v[c]);
+      add_if(s, c < nvalid && x > cut, x);
+      count += (c < nvalid && x > cut) ? 1 : 0;
     }
+    group_sums<G>(s, count);
+    sum = static_cast<R>(s);
+  };
+  above(-num<R>::inf());
+  const bool masked = sum == -num<R>::inf() || (count < m && sum < num<R>::inf());
+  R cut = -num<R>::inf();
+  if (masked) {
+    const R bound = lo + rho * (static_cast<R>(m) * lo);
+    cut = bound - fabs(bound) * (R(16) * num<R>::eps());
+    above(cut);
+  } else {
+    count = m;
+    const KnapState<R> st =
+        knap_equality<G, C, D, R, S, MAX_START>(v, m, nvalid, lo, hi, rhs);
+    if (st.t >= rho * rhs - eps)
+      return tag_thr(make_thr<R>(st.t_acc, lo, hi), SDCA_BRANCH_KNAPSACK, st.n_u, st.n_f);
   }
-  return tag_thr(make_thr<R>(st.t_acc, lo, hi),
-                 pp.op == OP_KNAPSACK_EQ ? SDCA_BRANCH_SEARCH : SDCA_BRANCH_KNAPSACK, st.n_u,
-                 st.n_f);
+  const R t = knapsack_biased_regs<G, C, D, R, S>(v, m, sum, lo, hi, rhs, R(1) / rho, cut,
+                                                  m - count);
+  if (!masked || t <= rho * rhs + eps) return tag_thr(make_thr<R>(t, lo, hi), SDCA_BRANCH_SCAN);
+  cut = lo + t;
+  above(cut);
+  const KnapState<R> st = knapsack_eq_regs<G, C, D, R, false, S>(
+      v, count, nvalid, sum, lo, hi, rhs - lo * static_cast<R>(m - count), num<R>::inf(), 0, R(0),
+      nullptr, nullptr, cut);
+  return tag_thr(make_thr<R>(st.t_acc, lo, hi), SDCA_BRANCH_KNAPSACK, st.n_u, st.n_f);
+}
+
+// ---------------------------------------------------------------------------
+// Knapsack family: knapsack_eq (knapsack_eq.h:25-109) and knapsack_le
+// (knapsack_le.h:17-44).  MAX_START: the start from the bound max - rhs above
+// (the prox kernels).  The SDCA epoch goes without it: its hinge takes that
+// start at k = 1 only, and carried its exchange buffer (1 KiB of LDS), up to
+// nine registers and the spilled scalars of its branch for every other k.
+// WIDE_BIASED: a workgroup's kernel for knapsack_le_biased with rho > 0; the
+// one for the other operators does without that code's registers (40e6 fp32
+// entries: m = 16000 341 -> 259 us, 30000 501 -> 395).
+// ---------------------------------------------------------------------------
+template <int G, int C, class D, class R, bool MAX_START = true, bool WIDE_BIASED = false>
+__device__ inline ColThr<R> knap_family(const D (&v)[C], int m, int nvalid,
+                                        const ProxParamsT<R>& pp) {
+  const R lo = pp.lo, hi = pp.hi, rhs = pp.rhs;
+  // Columns held by a workgroup of 512 threads or more carry their sums in
+  // WideSum and round them once, as the sorted column does (sum_range).  The
+  // float ones start from the mean: the rounding of the fixing's numerator
+  // (sums of thousands over a dozen free values) decides which values near t
+  // are free, and they take the sorted column's steps.
+  constexpr bool kWide = G >= 512;
+  typedef typename std::conditional<kWide, typename WideSum<R>::type, R>::type S;
+  constexpr bool kMaxStart = MAX_START && !(kWide && sizeof(R) == 4);
+  if constexpr (WIDE_BIASED) {
+    return knapsack_le_biased_wide<G, C, D, R, S, kMaxStart>(v, m, nvalid, pp);
+  } else {
+    // knapsack_le_biased with rho = 0 is knapsack_le (knapsack_le_biased.h:113-115).
+    const bool biased = !kWide && pp.op == OP_KNAPSACK_LE_BIASED && pp.rho != R(0);
+    if (pp.op == OP_KNAPSACK_LE || (pp.op == OP_KNAPSACK_LE_BIASED && !biased)) {
+      const R eps = num<R>::eps() * dmax(R(1), fabs(rhs));
+      S sum_mid = 0;
+      int n_hi = 0, n_mid = 0;
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        const R x = static_cast<R>(v[c]);
+        const bool up = x >= hi, mid = !up && x > lo;
+        add_if(sum_mid, mid, x);
+        n_hi += up ? 1 : 0;
+        n_mid += mid ? 1 : 0;
+      }
+      group_sums<G>(sum_mid, n_hi, n_mid);
+      const R s_mid = static_cast<R>(sum_mid);
+      const int n_lo = m - n_hi - n_mid;
+      const R s = s_mid + hi * static_cast<R>(n_hi) + lo * static_cast<R>(n_lo);
+      if (!(s > rhs + eps))
+        return tag_thr(make_thr<R>(R(0), lo, hi), SDCA_BRANCH_INACTIVE, n_hi, n_mid);
+    }
+    const KnapState<R> st = knap_equality<G, C, D, R, S, kMaxStart>(v, m, nvalid, lo, hi, rhs);
+    if (biased) {
+      // knapsack_le_biased.h:117-128: the equality solution stands if
+      // t >= rho rhs - eps; otherwise the sum constraint is inactive.
+      const R eps = num<R>::eps() * dmax(R(1), fabs(rhs));
+      if (!(st.t >= pp.rho * rhs - eps)) {
+        const R total = total_sum<G, C, D, R>(v, nvalid);
+        return tag_thr(make_thr<R>(knapsack_biased_regs<G, C, D, R>(v, m, total, lo, hi, rhs,
+                                                                    R(1) / pp.rho),
+                                   lo, hi),
+                       SDCA_BRANCH_SCAN);
+      }
+    }
+    return tag_thr(make_thr<R>(st.t_acc, lo, hi),
+                   pp.op == OP_KNAPSACK_EQ ? SDCA_BRANCH_SEARCH : SDCA_BRANCH_KNAPSACK, st.n_u,
+                   st.n_f);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -2026,7 +2047,7 @@ __device__ __forceinline__ void columns_tile(unsigned char* smem_raw, int m, int
   R tw = 0;
   unsigned wbits = 0;
   if constexpr (FAM == FAM_KNAP) {
-    th = knap_family<G, C, D, R>(v, m, nvalid, pp);
+    th = knap_family<G, C, D, R, true, KM == 1>(v, m, nvalid, pp);
   } else if constexpr (FAM == FAM_TOPK) {
     th = topk_family<G, C, KM, D, R>(v, m, nvalid, pp, col, lds_dummy);
   } else if constexpr (FAM == FAM_ENT) {

@@ -1,0 +1,60 @@
+"""Sums that are carried beyond the Result type and rounded once: of the
+columns a workgroup holds.  Against exactly rounded sums (math.fsum)."""
+import math
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def cancelling(n, m, seed):
+    """Columns whose large values cancel: the exact sum is about 1e-9 of the
+    values' magnitude."""
+    rng = np.random.default_rng(seed)
+    x = rng.standard_normal((n, m)) * 1e3
+    x[:, 1::2] = -x[:, 0:2 * (m // 2):2]
+    x[:, ::7] += rng.standard_normal((n, len(range(0, m, 7)))) * 1e-6
+    for j in range(n):
+        x[j] = x[j, rng.permutation(m)]
+    return x
+
+
+@pytest.mark.parametrize("m", [2049, 5000, 16384])
+@pytest.mark.parametrize("op,kw", [("knapsack_eq", {}), ("knapsack_le", {}),
+                                   ("knapsack_le_biased", dict(rho=0.5))])
+def test_knapsack_all_free(cuda, op, kw, m):
+    """Every value free: t = (sum a - rhs) / m (or sum a / (1 / rho + m))."""
+    import torch
+    import libsdca_amd as sd
+    x = cancelling(8, m, m)
+    s = np.array([math.fsum(c) for c in x])
+    rhs = 1e-8 if op == "knapsack_eq" else 0.0
+    if op == "knapsack_le":
+        x, s = np.where(s[:, None] < 0, -x, x), np.abs(s)  # the sum constraint acts
+    _, thr = sd.prox(op, torch.from_numpy(x).to(cuda), lo=-1e6, hi=1e6, rhs=rhs, thresholds=True,
+                     **kw)
+    t = thr.cpu().numpy()[:, 0]
+    want = (s - rhs) / m
+    if op == "knapsack_le_biased":
+        want = np.where(want >= 0, want, s / (2.0 + m))
+    # three roundings of terms no larger than |sum| + rhs, over m
+    u = np.finfo(np.float64).eps / 2
+    assert (np.abs(t - want) <= 6 * u * (np.abs(s) + rhs) / m).all()
+
+
+@pytest.mark.parametrize("m", [2049, 10000, 30000])
+def test_knapsack_le_inactive(cuda, m):
+    """knapsack_le's test of the sum constraint: the float sum is the exact
+    one rounded once (sums within a few ulps of the bound)."""
+    import torch
+    import libsdca_amd as sd
+    f32 = np.float32
+    rng = np.random.default_rng(m)
+    x = rng.random((64, m))
+    x = (x / x.sum(axis=1, keepdims=True) * (1 + rng.uniform(0, 3e-7, (64, 1)))).astype(f32)
+    _, sets = sd.prox("knapsack_le", torch.from_numpy(x).to(cuda), sets=True)
+    branch = [sd.BRANCHES[int(b)] for b in sets.cpu().numpy()[:, 2]]
+    active = np.array([f32(math.fsum(c)) > f32(1) + np.finfo(f32).eps for c in x])
+    assert 0 < active.sum() < 64
+    assert (np.array([b != "inactive" for b in branch]) == active).all()

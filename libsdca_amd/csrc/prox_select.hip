@@ -80,6 +80,10 @@ prox_select_kernel(const D* __restrict__ in, D* __restrict__ out, int64_t m64, i
   // thousands, a dozen values free, they place t a hundred ulps off, and a
   // result should not depend on the path its column takes.
   constexpr bool kClose = BT > 64 && sizeof(R) == 4;
+  // The sums over the column are rounded to R once, as the sorted column's.
+  typedef typename WideSum<R>::type S;
+  // (their loops unrolled further would set the kernel's register peak)
+  constexpr int UF = (sizeof(R) == 4 && BT > 64) ? 4 : 1;
   __shared__ R sh_mag[kClose ? BT / 64 : 1];
   const int grp = BT > 64 ? 0 : static_cast<int>(threadIdx.x) >> 6;
   const int lane = static_cast<int>(threadIdx.x) & 63;
@@ -289,17 +293,18 @@ prox_select_kernel(const D* __restrict__ in, D* __restrict__ out, int64_t m64, i
         // and the fixing below read the column again, from the L2: unrolled
         // over the slots they set the kernel's register peak.)
         const R eps16 = R(16) * num<R>::eps();
-        R s_p = 0;
+        S sum_p = 0;
         int n_p = 0, n_z = 0;
-#pragma unroll 4
+#pragma unroll UF
         for (int i = tid; i < m; i += BT) {
           const R x = static_cast<R>(col[i]);
           const bool pos = x > eps16;
-          s_p += pos ? x : R(0);
+          add_if(sum_p, pos, x);
           n_p += pos ? 1 : 0;
           n_z += (!pos && x >= -eps16) ? 1 : 0;
         }
-        group_sums<BT>(s_p, n_p, n_z);
+        group_sums<BT>(sum_p, n_p, n_z);
+        const R s_p = static_cast<R>(sum_p);
         const R K = static_cast<R>(k);
         const R hi = (K * s_p) / (K * K);
         const R largest = n_p > 0 ? static_cast<R>(list[0]) : -num<R>::inf();
@@ -331,7 +336,6 @@ prox_select_kernel(const D* __restrict__ in, D* __restrict__ out, int64_t m64, i
         // steps (knapsack_sorted: the same start, the numerator carried on
         // in R, the sums rounded to R once), so that it ends with the same
         // sets.
-        typedef typename std::conditional<(BT > 64), double, R>::type S;
         const R hi = pp.rhs_k, rhs = pp.rhs;
         const R eps = num<R>::eps() * dmax(R(1), fabs(rhs));
         R lc = -num<R>::inf(), hc = num<R>::inf();
@@ -343,30 +347,30 @@ prox_select_kernel(const D* __restrict__ in, D* __restrict__ out, int64_t m64, i
         }
         S s_f = 0, s_u = 0;
         int n_f = 0, n_u = 0;
-#pragma unroll 4
+#pragma unroll UF
         for (int i = tid; i < m; i += BT) {
           const R x = static_cast<R>(col[i]);
           const bool f = x > lc && x <= hc;
-          s_f += f ? x : R(0);
+          add_if(s_f, f, x);
           n_f += f ? 1 : 0;
-          s_u += x > hc ? x : R(0);
+          add_if(s_u, x > hc, x);
           n_u += x > hc ? 1 : 0;
         }
         group_sums<BT>(s_f, s_u, n_f, n_u);
         R t, t_fix;
         if constexpr (BT > 64) t = (static_cast<R>(s_f) - rhs) / static_cast<R>(n_f);
-        else t = div_near(s_f + static_cast<R>(n_u) * hi - rhs, static_cast<R>(n_f));
+        else t = (static_cast<R>(s_f) + static_cast<R>(n_u) * hi - rhs) / static_cast<R>(n_f);
         for (int iter = 0; iter <= m; ++iter) {
           const R c_hi = hi + t;
           S s_lo = 0, s_hi = 0;
           int n_lo = 0, n_hi = 0;
-#pragma unroll 4
+#pragma unroll UF
           for (int i = tid; i < m; i += BT) {
             const R x = static_cast<R>(col[i]);
             const bool f = x > lc && x <= hc;
-            s_lo += (f && x <= t) ? x : R(0);
+            add_if(s_lo, f && x <= t, x);
             n_lo += (f && x <= t) ? 1 : 0;
-            s_hi += (f && x > c_hi) ? x : R(0);
+            add_if(s_hi, f && x > c_hi, x);
             n_hi += (f && x > c_hi) ? 1 : 0;
           }
           group_sums<BT>(s_lo, s_hi, n_lo, n_hi);
@@ -394,16 +398,16 @@ prox_select_kernel(const D* __restrict__ in, D* __restrict__ out, int64_t m64, i
           }
           if (BT > 64 && (fix_hi || fix_lo)) continue;
           s_f = 0;
-#pragma unroll 4
+#pragma unroll UF
           for (int i = tid; i < m; i += BT) {
             const R x = static_cast<R>(col[i]);
-            s_f += (x > lc && x <= hc) ? x : R(0);
+            add_if(s_f, x > lc && x <= hc, x);
           }
           s_f = group_sum<BT>(s_f);
           if constexpr (BT > 64)
             t = (static_cast<R>(s_f) + static_cast<R>(n_u) * hi - rhs) / static_cast<R>(n_f);
           else
-            t = t_fix = div_near(s_f + static_cast<R>(n_u) * hi - rhs, static_cast<R>(n_f));
+            t = t_fix = (static_cast<R>(s_f) + static_cast<R>(n_u) * hi - rhs) / static_cast<R>(n_f);
           if (!fix_hi && !fix_lo) break;
         }
         bool lt;
@@ -411,7 +415,7 @@ prox_select_kernel(const D* __restrict__ in, D* __restrict__ out, int64_t m64, i
         if (n_u == 0) lt = t_fix < pp.rho * rhs - eps;
         else
           lt = K * (static_cast<R>(s_u) + (K - num_u) * t_fix) < rhs * (num_u + pp.rho * K * K) - eps;
-        const R sum_k = static_cast<R>(ps[k]);
+        const R sum_k = list_sum<R>(list, ps, 0, k);
         const bool constant =
             static_cast<R>(list[k - 1]) - sum_k / (K + pp.rho * K * K) >=
             static_cast<R>(k < cnt ? list[k] : list_rest(cut)) - R(16) * num<R>::eps();
@@ -565,7 +569,9 @@ hipError_t select_by_m(const ProxLaunch& a, bool all_columns) {
   if (a.m <= 2048) return select_one<D, R, 64, 32>(a, all_columns);
   if (a.m <= 4096) return select_one<D, R, 256, 16>(a, all_columns);
   if (a.m <= 8192) return select_one<D, R, 512, 16>(a, all_columns);
-  if (a.m <= 16384) return select_one<D, R, 1024, 16>(a, all_columns);
+  // (1024 threads of 16 slots spill: 128 registers.  m = 10,000: 4096 fp32
+  // columns 265 us so, 201 with 512 threads; 2000 fp64 columns 547, 88.)
+  if (a.m <= 16384) return select_one<D, R, 512, 32>(a, all_columns);
   if constexpr (sizeof(D) == 4) return select_one<D, R, 1024, 32>(a, all_columns);
   return hipErrorInvalidValue;
 }

@@ -143,6 +143,26 @@ __device__ inline D list_rest(D cut) {
   return cut > -num<D>::max_finite() ? cut : -num<D>::inf();
 }
 
+// The sum of the list's values [b, e) rounded to R once, in every lane: from
+// the prefix sums in double for float; for double compensated, a few values
+// one after the other (the lanes' six exchanges of pairs are a longer chain).
+template <class R, class D>
+__device__ inline SumPair list_sum_pair(const D* list, int b, int e) {
+  SumPair s = 0.0;
+  if (e - b <= 12) {
+    for (int i = b; i < e; ++i) s += static_cast<R>(list[i]);
+    return s;
+  }
+  for (int i = b + (static_cast<int>(threadIdx.x) & 63); i < e; i += 64)
+    s += static_cast<R>(list[i]);
+  return wave_total(s);
+}
+template <class R, class D>
+__device__ inline R list_sum(const D* list, const double* ps, int b, int e) {
+  if constexpr (sizeof(R) == 4) return static_cast<R>(ps[e] - ps[b]);
+  else return static_cast<R>(list_sum_pair<R>(list, b, e));
+}
+
 // The partition of the knapsack sum_i clamp(a_i - t, 0, hi) = rhs on the
 // sorted list (every value above t is in it): rank r is above t where
 // f(a_r) < rhs and at hi where f(a_r - hi) <= rhs, one rank per lane, f from
@@ -192,8 +212,12 @@ __device__ inline void list_knapsack(const D* list, const double* ps, int cnt, i
   if (u > e) u = e;
   if (e > u) {
     double s = 0;
-    for (int i = u + lane; i < e; i += 64) s += static_cast<double>(list[i]);
-    s = wave_total(s);
+    if constexpr (sizeof(R) == 4) {
+      for (int i = u + lane; i < e; i += 64) s += static_cast<double>(list[i]);
+      s = wave_total(s);
+    } else {
+      s = list_sum<R>(list, ps, u, e);
+    }
     t_out = static_cast<R>((s + static_cast<double>(u) * hi - rhs) / static_cast<double>(e - u));
   } else {
     const double top = (u > 0 ? static_cast<double>(list[u - 1]) : static_cast<double>(list[0])) - hi;
@@ -204,6 +228,32 @@ __device__ inline void list_knapsack(const D* list, const double* ps, int cnt, i
   }
   u_out = u;
   e_out = e;
+}
+
+// t = (nu sum_M - k_u sum_U) / den and hi = (|M| sum_U + k_u sum_M) / den of
+// the partition U = [0, u), M = [u, e), whose terms may cancel: in double for
+// float; for double from compensated sums, the products' rounding kept (fma).
+template <class D>
+__device__ inline void list_cone_values(const D*, const double* ps, int u, int e, float k_u,
+                                        float nu, float& t, float& hi) {
+  const double su = ps[u], sm = ps[e] - su;
+  const double ku = k_u, n = nu, n_m = e - u, den = ku * ku + n_m * n;
+  t = static_cast<float>(div_near(n * sm - ku * su, den));
+  hi = static_cast<float>(div_near(n_m * su + ku * sm, den));
+}
+__device__ inline double two_products(double a, const SumPair& x, double b, const SumPair& y) {
+  const double p = a * x.s, q = b * y.s;
+  SumPair r(p);
+  r += q;
+  return r.s + (r.c + ((fma(a, x.s, -p) + fma(b, y.s, -q)) + (a * x.c + b * y.c)));
+}
+template <class D>
+__device__ inline void list_cone_values(const D* list, const double*, int u, int e, double k_u,
+                                        double nu, double& t, double& hi) {
+  const SumPair su = list_sum_pair<double>(list, 0, u), sm = list_sum_pair<double>(list, u, e);
+  const double n_m = e - u, den = k_u * k_u + n_m * nu;
+  t = two_products(nu, sm, -k_u, su) / den;
+  hi = two_products(n_m, su, k_u, sm) / den;
 }
 
 // topk_cone_search (topk_cone.h:58-133) and its biased form
@@ -248,11 +298,9 @@ __device__ inline SelectRecord<R> list_cone(const D* list, const double* ps, int
       const bool take = pass && (ei == m || next - eps <= t);
       const unsigned long long taken = __ballot(take);
       if (taken) {
-        const int l = __ffsll(taken) - 1;
-        rec.t = read_lane(t, __builtin_amdgcn_readfirstlane(l));
-        rec.hi = read_lane(hi, __builtin_amdgcn_readfirstlane(l));
         rec.n_hi = u;
-        rec.n_mid = e0 + l - u;
+        rec.n_mid = e0 + __ffsll(taken) - 1 - u;
+        list_cone_values(list, ps, u, u + rec.n_mid, k_u, nu, rec.t, rec.hi);
         return rec;
       }
       // Nothing accepted up to e: where t is certainly above every later
@@ -296,7 +344,7 @@ __device__ inline SelectRecord<R> list_record(const D* list, const double* ps, i
   rec.branch = SDCA_BRANCH_ZERO;
   rec.n_hi = rec.n_mid = 0;
   if (cnt < k) return rec;  // masked classes among the k largest: no sum above 0
-  const R sum_k = static_cast<R>(ps[k]);
+  const R sum_k = list_sum<R>(list, ps, 0, k);
   if (sum_k <= eps16) return rec;
   const R hi_c = sum_k / (K + rho * K * K);
   const R t_c = static_cast<R>(list[k - 1]) - hi_c;
@@ -323,7 +371,7 @@ __device__ inline SelectRecord<R> list_record(const D* list, const double* ps, i
         lt = rec.t < rho * rhs - eps;
       } else {
         const R num_u = static_cast<R>(u);
-        lt = K * (static_cast<R>(ps[u]) + (K - num_u) * rec.t) < rhs * (num_u + rho * K * K) - eps;
+        lt = K * (list_sum<R>(list, ps, 0, u) + (K - num_u) * rec.t) < rhs * (num_u + rho * K * K) - eps;
       }
     }
     if (!lt) {

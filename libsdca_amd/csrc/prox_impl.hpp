@@ -296,7 +296,10 @@ __device__ inline KnapState<R> knapsack_eq_regs(const D (&v)[C], int m, int nval
 template <int G, int C, class D, class R, class S = R>
 __device__ inline R knapsack_biased_regs(const D (&v)[C], int m, R total, R lo, R hi, R rhs,
                                          R rho_inv, R floor = -num<R>::inf(), int n_floor = 0) {
-  const R eps = num<R>::eps() * dmax(R(1), fabs(rhs));
+  // (eps = max(1, rhs) eps passes over candidates whose excess it hides: for
+  // values of size 1e-3 that leaves t 3 ulps off.  The search over the sorted
+  // column, which S wider than R stands for, has no such tolerance.)
+  const R eps = sizeof(S) > sizeof(R) ? R(0) : num<R>::eps() * dmax(R(1), fabs(rhs));
   const R qnan = num<R>::quiet_nan();
   int n_l = n_floor, n_u = 0;
   R s_free = total;

@@ -58,3 +58,23 @@ def test_knapsack_le_inactive(cuda, m):
     active = np.array([f32(math.fsum(c)) > f32(1) + np.finfo(f32).eps for c in x])
     assert 0 < active.sum() < 64
     assert (np.array([b != "inactive" for b in branch]) == active).all()
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("m", [2049, 3000, 16384])
+def test_knapsack_le_biased_small_values(cuda, m, dtype):
+    """The search's t = rho sum x on values of size 1e-3, far below the
+    tolerance the sum constraint's size gives."""
+    import torch
+    import libsdca_amd as sd
+    n = 64 if m > 5000 else 400
+    x = (np.random.default_rng(m).standard_normal((n, m)) * 1e-3).astype(dtype)
+    _, thr = sd.prox("knapsack_le_biased", torch.from_numpy(x).to(cuda), rho=0.5, thresholds=True)
+    t = thr.cpu().numpy()[:, 0]
+    want = np.empty(n)
+    for j in range(n):  # sum of the n largest over 1 / rho + n, the n that are above it
+        a = np.sort(x[j].astype(np.longdouble))[::-1]
+        r = np.cumsum(a) / (2 + np.arange(1, m + 1))
+        want[j] = r[int((a > r).sum()) - 1]
+    # the sum's and the quotient's rounding: 2 ulps
+    assert (np.abs(t - want) <= 2 * np.finfo(dtype).eps * want).all()

@@ -135,9 +135,9 @@ struct KnapState {
 // their stores go to the lane's dummy word) instead of C more registers.
 // The caller must not need the LDS copy of the column afterwards.
 //
-// S: the type every pass's sums are carried in (R, or WideSum<R>: rounded to
-// R once).
-template <int G, int C, class D, class R, bool WL = false, class S = R>
+// S: the type the final free set's sum is carried in, SP every pass's sums (R,
+// or WideSum<R>: rounded to R once).
+template <int G, int C, class D, class R, bool WL = false, class S = R, class SP = S>
 __device__ inline KnapState<R> knapsack_eq_regs(const D (&v)[C], int m, int nvalid, R total,
                                                 R lo, R hi, R rhs, R hi_cut0 = num<R>::inf(),
                                                 int n_u0 = 0, R sum_u0 = 0, D* wl = nullptr,
@@ -167,7 +167,7 @@ __device__ inline KnapState<R> knapsack_eq_regs(const D (&v)[C], int m, int nval
   // own roundings (knapsack_sorted), so that both end with the same sets.
   constexpr bool SEQ = sizeof(S) > sizeof(R);
   auto quotient = [](R n, R d) -> R {
-    if constexpr (SEQ) return n / d;
+    if constexpr (sizeof(SP) > sizeof(R)) return n / d;
     else return div_near(n, d);
   };
   int mc = m - n_u0;
@@ -189,7 +189,7 @@ __device__ inline KnapState<R> knapsack_eq_regs(const D (&v)[C], int m, int nval
   }
   for (int iter = 0; iter <= m; ++iter) {
     const R c_lo = lo + t, c_hi = hi + t;
-    S sum_lo = 0, sum_hi = 0;
+    SP sum_lo = 0, sum_hi = 0;
     int n_lh = 0;
 #pragma unroll UW
     for (int c = 0; c < C; ++c) {
@@ -732,7 +732,8 @@ __device__ inline void group_sort_desc(D (&x)[CC], int g) {
 // k hi against rhs.  Returns false, for the variable fixing to decide, when
 // no u fits (ties with a threshold at rounding level), hi <= 0 or a value
 // is not finite.
-template <int G, int CC, int L, class D, class R>
+// S: the type the sums that end in the record are carried in.
+template <int G, int CC, int L, class D, class R, class S = R>
 __device__ inline bool topk_sorted_root(const D* lds_col, int total, const D (&top)[L], int k,
                                         R hi, R rhs, KnapState<R>& st) {
   constexpr int N = G * CC;
@@ -822,14 +823,15 @@ __device__ inline bool topk_sorted_root(const D* lds_col, int total, const D (&t
   if (u >= 0) {
     // The threshold applied, from the sum over M taken directly; the sets
     // as value cuts (U = values above a_u, M = the rest above a_e).
-    R sm = 0;
+    S sum_m = 0;
 #pragma unroll
     for (int c = 0; c < CC; ++c) {
       const int r = g * CC + c;
-      sm += (r >= u && r < e) ? static_cast<R>(x[c]) : R(0);
+      add_if(sum_m, r >= u && r < e, static_cast<R>(x[c]));
     }
-    sm = group_sum<G>(sm);
-    const R t = div_near(sm + static_cast<R>(u) * hi - rhs, static_cast<R>(e - u));
+    const R sm = static_cast<R>(group_sum<G>(sum_m));
+    const R num_m = sm + static_cast<R>(u) * hi - rhs, n_m = static_cast<R>(e - u);
+    const R t = sizeof(S) > sizeof(R) ? num_m / n_m : div_near(num_m, n_m);
     R su = 0, au = 0;
 #pragma unroll
     for (int j = 0; j < L - 1; ++j) {
@@ -882,7 +884,8 @@ __device__ inline bool topk_sorted_root(const D* lds_col, int total, const D (&t
 // candidates for the registers, the fixing over every slot keeps its working
 // copy in those LDS words (for callers where that case is rare and the
 // registers set the occupancy) rather than in C more registers.
-template <int G, int C, int L, class D, class R, bool LDS_FALLBACK>
+// S: the type the final free set's sum is carried in.
+template <int G, int C, int L, class D, class R, bool LDS_FALLBACK, class S = R>
 __device__ inline KnapState<R> topk_knapsack(const D (&v)[C], const D (&top)[L], int m,
                                              int nvalid, int k, R kth, R hi, R rhs, D* lds_col,
                                              D* lds_dummy, bool lane_lists = false) {
@@ -952,7 +955,7 @@ __device__ inline KnapState<R> topk_knapsack(const D (&v)[C], const D (&top)[L],
       group_lds_sync<G>();
       if constexpr (G == 4) {
         KnapState<R> st;
-        if (topk_sorted_root<G, CC, L, D, R>(lds_col, total, top, k, hi, rhs, st)) return st;
+        if (topk_sorted_root<G, CC, L, D, R, S>(lds_col, total, top, k, hi, rhs, st)) return st;
       }
       // Candidate i sits at lds_col[i]; lane g takes i = g, g + G, ...  The
       // reads stay inside the tile: G * CC <= 16 <= m for G = 4 and 2, and
@@ -979,8 +982,8 @@ __device__ inline KnapState<R> topk_knapsack(const D (&v)[C], const D (&top)[L],
         n_u0 += u ? 1 : 0;
         sum_u0 += u ? static_cast<R>(top[i]) : R(0);
       }
-      return knapsack_eq_regs<G, CC, D, R>(cand, total, total, csum, R(0), hi, rhs, ucut, n_u0,
-                                           sum_u0);
+      return knapsack_eq_regs<G, CC, D, R, false, S, R>(cand, total, total, csum, R(0), hi, rhs,
+                                                        ucut, n_u0, sum_u0);
     }
     if constexpr (G > 64) {
       // More candidates than registers on a workgroup-wide group (the
@@ -1006,7 +1009,7 @@ __device__ inline KnapState<R> topk_knapsack(const D (&v)[C], const D (&top)[L],
     }
   }
   const R all = total_sum<G, C, D, R>(v, nvalid);
-  return knapsack_eq_regs<G, C, D, R, (LDS_FALLBACK && G > 1)>(
+  return knapsack_eq_regs<G, C, D, R, (LDS_FALLBACK && G > 1), S, R>(
       v, m, nvalid, all, R(0), hi, rhs, num<R>::inf(), 0, R(0),
       lds_col + static_cast<int>(threadIdx.x) % G, lds_dummy);
 }
@@ -1023,6 +1026,10 @@ __device__ inline ColThr<R> topk_family(const D (&v)[C], int m, int nvalid,
   const R K = static_cast<R>(k);
   const R eps16 = R(16) * num<R>::eps();
   constexpr int L = KM + 1;
+  // The longest list's kernels took the columns of the sorted form, which
+  // rounds its sums to R once: so do they where the sums end in the record.
+  // (Not the epoch's, LDS_FALLBACK = false.)
+  typedef typename std::conditional<(KM == 15 && LDS_FALLBACK), typename WideSum<R>::type, R>::type S;
   D top[L];
 #pragma unroll
   for (int i = 0; i < L; ++i) top[i] = -num<D>::inf();
@@ -1047,13 +1054,15 @@ __device__ inline ColThr<R> topk_family(const D (&v)[C], int m, int nvalid,
     for (int i = 0; i < L; ++i) lds_col[g * L + i] = top[i];
   }
   top_merge<G>(top);
-  R sum_k = 0, kth = static_cast<R>(top[0]), next = -num<R>::inf();
+  S top_sum = 0;
+  R kth = static_cast<R>(top[0]), next = -num<R>::inf();
 #pragma unroll
   for (int i = 0; i < L; ++i) {
-    if (i < k) sum_k += static_cast<R>(top[i]);
+    if (i < k) top_sum += static_cast<R>(top[i]);
     if (i == k - 1) kth = static_cast<R>(top[i]);
     if (i == k) next = static_cast<R>(top[i]);
   }
+  const R sum_k = static_cast<R>(top_sum);
   const R largest = static_cast<R>(top[0]);
   // topk_cone_special_cases (topk_cone.h:18-55), whose divisor is k, or
   // k + rho k^2 for the biased simplex (topk_simplex_biased.h:50-51).
@@ -1079,9 +1088,9 @@ __device__ inline ColThr<R> topk_family(const D (&v)[C], int m, int nvalid,
   const R hi = pp.rhs_k;  // rhs / K (topk_simplex.h:56)
   // More than G * kCandSlots candidates is rare for the prox inputs: the LDS
   // working copy keeps the kernel's register peak at the candidate path's.
-  KnapState<R> st = topk_knapsack<G, C, L, D, R, LDS_FALLBACK>(v, top, m, nvalid, k, kth, hi,
-                                                                rhs, lds_col, lds_dummy,
-                                                                lane_lists);
+  KnapState<R> st = topk_knapsack<G, C, L, D, R, LDS_FALLBACK, S>(v, top, m, nvalid, k, kth, hi,
+                                                                   rhs, lds_col, lds_dummy,
+                                                                   lane_lists);
   if (!constant) {
     // is_topk_simplex_lt (topk_simplex.h:9-27), is_topk_simplex_biased_lt
     // (topk_simplex_biased.h:9-28), over U = [first, t.first)

@@ -78,3 +78,28 @@ def test_knapsack_le_biased_small_values(cuda, m, dtype):
         want[j] = r[int((a > r).sum()) - 1]
     # the sum's and the quotient's rounding: 2 ulps
     assert (np.abs(t - want) <= 2 * np.finfo(dtype).eps * want).all()
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("m", [16, 40, 100, 200, 300, 512, 700, 3000])
+def test_topk_constant(cuda, m, dtype):
+    """The k = 12 largest equal by the projection, hi = (sum of them) / 12,
+    where large values cancel in that sum."""
+    import torch
+    import libsdca_amd as sd
+    k = 12
+    rng = np.random.default_rng(m)
+    x = np.full((50, m), -1e5)
+    for j in range(50):
+        # (their sum is 8 ulps of a value of 100 at least: above 16 eps, where
+        # the zero branch ends)
+        a = rng.uniform(100, 1000, k // 2).astype(np.float32)
+        top = np.concatenate([a, -a[:-1], [-a[-1] + np.spacing(a[-1], dtype=np.float32) * 8]])
+        x[j, rng.permutation(m)[:k]] = top
+    x = x.astype(dtype)
+    for op, kw, div in (("topk_cone", {}, 12.0), ("topk_cone_biased", dict(rho=0.25), 12 + 0.25 * 144)):
+        _, thr = sd.prox(op, torch.from_numpy(x).to(cuda), k=k, thresholds=True, **kw)
+        hi = thr.cpu().numpy()[:, 2]
+        want = np.array([math.fsum(sorted(c)[-k:]) for c in x]) / div
+        # the sum's rounding and the quotient's
+        assert (np.abs(hi - want) <= 2 * np.finfo(dtype).eps * want).all(), op

@@ -192,7 +192,8 @@ int sdca_prox_with_sets(sdca_prox_op op, sdca_dtype data, sdca_dtype result,
  * biased and sort-based two-simplex operators lives in a fixed device array
  * of the library, one per device, held until the process ends: those
  * operators take at most sdca_prox_noalloc_max_columns() columns (4,194,304)
- * per call and return SDCA_ERR_ARG_RANGE beyond; the other operators use no
+ * per call and return SDCA_ERR_ARG_RANGE beyond (the biased knapsack too,
+ * although it defers no column); the other operators use no
  * scratch and take any n.  Every call on a device shares that array: calls
  * that overlap on one device (concurrent streams or host threads) race.
  */

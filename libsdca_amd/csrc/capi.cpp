@@ -291,9 +291,9 @@ int prox_entry(int op_in, int data_in, int result_in, int64_t m, int64_t n, cons
 
   const bool reg_ok = m <= kRegMaxM;
   const bool topk = op == SDCA_PROX_TOPK_SIMPLEX || op == SDCA_PROX_TOPK_CONE;
-  // The biased simplex, cone and knapsack run in the register kernel;
-  // columns whose search needs more of the sorted column are deferred to the
-  // workgroup-per-column kernel through the column list.
+  // The biased simplex, cone and knapsack run in the register kernel; the
+  // simplex's and cone's columns whose search needs more of the sorted column
+  // are deferred to the selection kernel through the column list.
   const bool reg_biased = op == SDCA_PROX_TOPK_SIMPLEX_BIASED ||
                           op == SDCA_PROX_TOPK_CONE_BIASED || op == SDCA_PROX_KNAPSACK_LE_BIASED;
   const bool topk_like =

@@ -226,10 +226,12 @@ hipError_t launch_primal_t(const void* X, const void* A, const void* W0, void* W
 // to 256 classes, the library's transposed copies costing more than its
 // GEMM gains (n = 100,000: m = 18, d = 3207 1150 -> 717 us; m = 200, d =
 // 1024 1045 -> 738; m = 1000 stays).  fp64 sums over more than 65,536
-// examples keep the one running sum of the score GEMM: splitting them moves
-// W by more than 1e-14 of its norm (3.4e-17 sqrt(n) measured).  The split
-// sums are the closer ones: n = 20,011, m = 137, d = 513 against long double,
-// 4.7e-15 of W's norm as one running sum, 7.6e-16 split.
+// examples keep the one running sum of the score GEMM, for agreement with the
+// W they always gave, which split sums would move by that sum's own error:
+// more than 1e-14 of its norm.  Neither time nor accuracy asks for it (m =
+// 137, d = 513, from long double in brackets: n = 65,536 split 452 us
+// [1.2e-15]; 70,000 kept 2992 [8.2e-15], split 472 [1.8e-15]; 200,000 kept
+// 8527 [1.6e-14], split 1334 [2.1e-15]).
 bool primal_split(int data, int64_t d, int64_t m, int64_t n) {
   const int64_t tiles = ((d + kTile - 1) / kTile) * ((m + kTile - 1) / kTile);
   if (tiles >= 512) return false;

@@ -3,8 +3,9 @@
 // capture, serving loops, harnesses that forbid hipMalloc).
 //
 // The only device memory sdca_prox allocates beyond its inputs and outputs
-// is the deferred-column list of the top-k, biased and sort-based
-// two-simplex operators: [count, done, column ids...], n + 2 ints.  Here it
+// is the deferred-column list of the top-k (biased or not) and sort-based
+// two-simplex operators: [count, done, column ids...], n + 2 ints.  (The
+// biased knapsack uses no list, but keeps their limit of columns.)  Here it
 // lives in the file-scope array below, one copy per device, which each
 // device holds until the process ends.  Its address on a device is looked up
 // once (hipGetSymbolAddress, with that device current) and cached; kernels

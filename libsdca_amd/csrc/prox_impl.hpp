@@ -18,9 +18,10 @@
 // of the reference expressed as value cuts (a partition by `x > c` keeps a
 // set {x > cut}).  Sums run in a different order than the reference's
 // std::accumulate, so thresholds agree to rounding.  Columns whose case needs
-// the reference's full sort (topk_cone_search with |U| > 0, ties at zero,
-// k beyond the register list) are flagged into a list that the
-// workgroup-per-column kernel in prox_slow.hip finishes.
+// more of the sorted column (topk_cone_search with |U| > 0, ties at zero, the
+// biased cone's scan past its list) are flagged into a list that the
+// selection kernel (prox_select.hip) finishes; two_simplex_sort's go to its
+// sort-and-scan kernel (prox_slow.hip).
 #ifndef SDCA_HIP_PROX_IMPL_HPP
 #define SDCA_HIP_PROX_IMPL_HPP
 
@@ -49,7 +50,7 @@ struct ColThr {
   R t, lo, hi;     // first (or only) block
   R t2, lo2, hi2;  // second block (two-block operator)
   int kind;        // elementwise map of the clamp: 0 identity, 1 exp, 2 W(exp)
-  bool slow;       // column deferred to the workgroup-per-column kernel
+  bool slow;       // column deferred to the list's kernel
   // The record's sets (sdca_prox_sets) and the branch that produced it:
   // n_hi < 0 leaves them to be counted from the column by the record's cuts
   // (x > t + hi at hi, x > t + lo free); n_mid2 is block b's free count (its
@@ -518,7 +519,7 @@ __device__ inline ColThr<R> knap_family(const D (&v)[C], int m, int nvalid,
 // topk_cone_search (topk_cone.h:58-133) when the answer has U empty: then
 // t = 0 exactly, M = {x > 16 eps} and hi = k sum(M) / k^2; valid if
 // hi >= max(M) - 16 eps.  Any other outcome (U non-empty, or values within
-// 16 eps of zero that the reference may place in M) goes to the slow path.
+// 16 eps of zero that the reference may place in M) is deferred.
 template <int G, int C, class D, class R>
 __device__ inline ColThr<R> cone_search_u0(const D (&v)[C], R K, R largest) {
   const R eps16 = R(16) * num<R>::eps();
@@ -1102,8 +1103,8 @@ __device__ inline ColThr<R> topk_family(const D (&v)[C], int m, int nvalid,
         const R num_u = static_cast<R>(st.n_u);
         lt = K * (st.sum_u + (K - num_u) * st.t) < rhs * (num_u + pp.rho * K * K) - eps;
       }
-      // The biased cone search (topk_cone_biased.h:58-137) runs on the
-      // sorted column in the workgroup-per-column kernel.
+      // The biased cone search (topk_cone_biased.h:58-137) runs in the
+      // selection kernel.
       if (lt) return slow_thr<R>();
     } else {
       if (st.n_u == 0) {
@@ -2074,7 +2075,7 @@ __device__ __forceinline__ void columns_tile(unsigned char* smem_raw, int m, int
   // The threshold search may have used the column's LDS slots as scratch.
   __syncthreads();
   if (active) {
-    // Deferred columns keep their input: the workgroup-per-column kernel
+    // Deferred columns keep their input: the list's kernel
     // reads it again (in place when in == out).  For the clamp-only families
     // that is the clamp with t = 0, lo = -inf, hi = +inf; the entropic maps
     // select the input instead.

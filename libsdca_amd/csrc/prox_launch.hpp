@@ -33,8 +33,8 @@ constexpr int64_t kRegMaxM = 2048;
 constexpr int kWideThreads = 512;
 constexpr int kMaxWideThreads = 1024;
 // Largest column (m times the element size) any kernel holds in LDS: the
-// sorted-column, wave-per-column and workgroup-per-column kernels stage
-// whole columns (160 KiB of LDS per workgroup on gfx950, less the dummy
+// sorted-column, wave-per-column and workgroup-per-column (wide register and
+// selection) kernels stage whole columns (160 KiB of LDS per workgroup on gfx950, less the dummy
 // words and reduction scratch).
 constexpr int64_t kMaxColumnBytes = 128 * 1024;
 // Largest m of the prox operators (and of the evaluation) for an element

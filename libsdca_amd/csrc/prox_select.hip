@@ -22,15 +22,15 @@
 // that the fixed work per column (two sorts of 64 values, the searches).
 // Measured on MI355X, 40e6 fp32 entries, us per launch, sorting the whole
 // column -> selection:
-//   top-k simplex k = 10:  m = 700 2568 -> 92, 1000 1875 -> 70, 1500 2261 -> 64
-//   top-k simplex k = 5, 4096 columns of 10,000:  7364 -> 296
+//   top-k simplex k = 10:  m = 700 2568 -> 92, 1000 1875 -> 68, 1500 2261 -> 63
+//   top-k simplex k = 5, 4096 columns of 10,000:  7364 -> 201
 //   top-k cone k = 5 on margins (U/M searches):  m = 100 12812 -> 653,
 //                          1000 15076 -> 443, 3000 7918 -> 105
 // (one read and one write of them take 52 us at the rate of a large copy
-// kernel).  A column that the list cannot decide (more than kSelectMax values above the cut and no
-// plain knapsack, values that are not finite, ties with zero, a partition
-// that may reach past the list) is sorted whole by the group that holds it
-// (prox_sorted.hpp).
+// kernel).  A column that the list cannot decide (more than kSelectMax values
+// above the cut and no plain knapsack, +inf or NaN, ties with zero, a
+// partition that may reach past the list) is sorted whole by the group that
+// holds it (prox_sorted.hpp).  Classes masked by -inf are left out.
 #include <algorithm>
 #include <climits>
 #include <type_traits>

@@ -7,7 +7,8 @@
 // by one wave, with the reference's tests in its order; the partitions are
 // found by binary search and the range sums by the wave's 64 lanes
 // (compensated), the scans' incremental sums in the reference's order.  Used
-// by the workgroup-per-column prox kernel and the SDCA epoch.
+// by the sorted-column prox kernel, the selection kernel's fallback, the
+// evaluation's deferred examples and the SDCA epoch.
 #ifndef SDCA_HIP_PROX_SORTED_HPP
 #define SDCA_HIP_PROX_SORTED_HPP
 

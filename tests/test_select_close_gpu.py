@@ -80,3 +80,23 @@ def test_close_call(cuda, m, k):
     want = np.clip(x - t[:, None], 0, np.float32(1))
     got, _ = run_gpu("knapsack_eq", x, F32, cuda, lo=0.0, hi=1.0, rhs=1.0)
     assert np.abs(got - want).max() <= tol
+
+
+@pytest.mark.parametrize("m,k", [(2049, 5), (4100, 10), (10000, 3), (20000, 1), (32768, 10)])
+def test_close_call_projection(cuda, oracle, m, k):
+    """How far those steps are from the projection (long double): the fixing's
+    numerator is rounded to float in each of its passes, of which there are at
+    most 16 here (the free set halves in each), by u sum |a| at most, over the
+    values free at the end."""
+    from oracle import binding
+    x = close_columns(m, k, 24, 900 + m + k)
+    u = np.finfo(np.float32).eps / 2
+    for op, kw in (("topk_simplex", dict(k=k, rhs=1.0)), ("knapsack_eq", dict(lo=0.0, hi=1.0, rhs=1.0))):
+        got, _ = run_gpu(op, x, F32, cuda, **kw)
+        want = x.astype(np.float64)
+        oracle.prox(op, want, result=2, params=binding.make_params(**kw), nthreads=8)
+        free = ((want > 0) & (want < (1.0 / k if op == "topk_simplex" else 1.0))).sum(axis=1)
+        bound = 16 * u * np.abs(x.astype(np.float64)).sum(axis=1) / np.maximum(free, 1)
+        err = np.abs(got - want).max(axis=1)
+        print(f"{op} m={m} k={k}: error {err.max():.1e}, at most {(err / bound).max():.2f} of the bound")
+        assert (err <= bound).all()

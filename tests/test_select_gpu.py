@@ -1,5 +1,5 @@
-"""The top-k operators by selection (prox_select.hip) against the CPU oracle: the sizes around each configuration step, k
-around the register lists, inputs that take every way through the selection
+"""The top-k operators by selection (prox_select.hip) against the CPU oracle:
+the sizes around each configuration step, k around the register lists, inputs that take every way through the selection
 (short lists, more candidates than the list holds, searches past the first
 list, ties with zero and with the thresholds, whole-column fallback)."""
 import numpy as np
@@ -78,8 +78,9 @@ def test_select_unaligned_and_in_place(cuda, oracle, k):
 
 
 def test_select_values_not_finite(cuda):
-    """A column that holds an infinity or a NaN is sorted whole, as before;
-    the others of the launch are not touched by it."""
+    """Columns that hold +inf, NaN (sorted whole; no projection is defined) or
+    -inf (a masked class: test_masked_gpu.py) do not touch the others of the
+    launch."""
     import torch
     import libsdca_amd as sd
     for m, k in ((300, 20), (3000, 5)):

@@ -479,10 +479,21 @@ __device__ inline ColThr<R> knap_family(const D (&v)[C], int m, int nvalid,
 #pragma unroll
       for (int c = 0; c < C; ++c) {
         const R x = static_cast<R>(v[c]);
-        const bool up = x >= hi, mid = !up && x > lo;
-        add_if(sum_mid, mid, x);
-        n_hi += up ? 1 : 0;
-        n_mid += mid ? 1 : 0;
+        // (Branches in a workgroup's kernel, selects in a wave's: m = 16000
+        // fp32 259 us against 336, m = 200 fp64 72 against 81.)
+        if constexpr (kWide) {
+          if (x >= hi) {
+            ++n_hi;
+          } else if (x > lo) {
+            sum_mid += x;
+            ++n_mid;
+          }
+        } else {
+          const bool up = x >= hi, mid = !up && x > lo;
+          add_if(sum_mid, mid, x);
+          n_hi += up ? 1 : 0;
+          n_mid += mid ? 1 : 0;
+        }
       }
       group_sums<G>(sum_mid, n_hi, n_mid);
       const R s_mid = static_cast<R>(sum_mid);

@@ -479,9 +479,10 @@ __device__ inline ColThr<R> knap_family(const D (&v)[C], int m, int nvalid,
 #pragma unroll
       for (int c = 0; c < C; ++c) {
         const R x = static_cast<R>(v[c]);
-        // (Branches in a workgroup's kernel, selects in a wave's: m = 16000
-        // fp32 259 us against 336, m = 200 fp64 72 against 81.)
-        if constexpr (kWide) {
+        // (Branches in a workgroup's kernel and in float, selects in a wave's
+        // double one: m = 16000 fp32 259 us against 336, m = 200 fp32 68
+        // against 72, fp64 81 against 72.)
+        if constexpr (kWide || sizeof(R) == 4) {
           if (x >= hi) {
             ++n_hi;
           } else if (x > lo) {
